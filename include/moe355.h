@@ -54,7 +54,8 @@ extern "C" {
 /* Kernel family chosen for the expert FFN. */
 #define MOE355_PATH_MFMA_TILED 0 /* 256x256 bf16/f16 MFMA tiles, prefill-sized groups */
 #define MOE355_PATH_MFMA_SKINNY 1 /* weight-streaming 16x16x32 MFMA, decode-sized groups */
-#define MOE355_PATH_SIMT 2        /* fp32 FMA tiles: fp32 layers and unaligned shapes */
+#define MOE355_PATH_SIMT 2        /* fp32 layers and sizes the other families do not take: MFMA tiles
+                                     (fp32 MFMA for fp32) of 16 or 64 token rows */
 /* 3 is unused (a 256x64-tile family that no workload chose was removed) */
 #define MOE355_PATH_MFMA_TILED128 4 /* the 256x256 kernel on 128-row token tiles, groups of ~128 rows */
 
@@ -172,7 +173,8 @@ int moe355_topk_from_logits(const float* logits, int T, int E, int K, int renorm
  * projection's K-split, and launches nothing. The kernel family follows the
  * average rows per active expert (T*K / min(T*K, E)): up to 10 skinny, up to
  * 104 the tiled kernel on 128-row tiles, above it 256-row tiles; fp32 and
- * shapes the MFMA kernels do not tile take the SIMT family. */
+ * sizes these kernels do not take run MOE355_PATH_SIMT, on 16-row tiles up to
+ * 10 rows and 64-row tiles above. */
 int moe355_make_plan(int T, int H, int I, int E, int K, int dtype, moe355_plan* plan);
 
 /* moe355_make_plan with the kernel family forced (`path` = MOE355_PATH_*, or -1
@@ -252,7 +254,7 @@ int moe355_fused_experts(const void* x, const void* const* w1, const void* const
  * Limits: a shape whose plan needs more than MOE355_STATIC_SCRATCH_BYTES
  * fails with MOE355_EWORKSPACE before launching anything (the tiled paths
  * first drop their down-projection partial tiles, running that projection's
- * last round whole). The calling thread's current device must be the device
+ * last round whole; MOE355_PATH_SIMT first drops its K-splits). The calling thread's current device must be the device
  * of `stream`. Every call on one device shares that device's array: calls
  * that overlap on one device (other streams, other threads) race and must
  * be serialised by the caller. Nothing in the array needs to start zeroed.

@@ -37,6 +37,9 @@ int check_hip(hipError_t e, const char* what) {
 
 constexpr int kMaxDevices = 64;
 
+// Average rows per active expert up to which 16-row weight-streaming tiles run.
+constexpr int kSkinnyRows = 10;
+
 size_t align256(size_t v) { return (v + 255) & ~static_cast<size_t>(255); }
 
 bool valid_dtype(int d) { return d == MOE355_F32 || d == MOE355_BF16 || d == MOE355_F16; }
@@ -95,6 +98,39 @@ int device_cu_count() {
 
 }  // namespace moe355
 
+namespace {
+
+int plan_impl(int T, int H, int I, int E, int K, int dtype, int path, bool compact,
+              moe355_plan* p);
+
+// Bytes of one operand row per K step of the general path's kernels: 256 in
+// ffn_skinny_kernel (16-row tiles), 128 in ffn_general_kernel (64-row tiles).
+int general_step_bytes(const moe355_plan* p) { return p->tile_rows == 16 ? 256 : 128; }
+
+// Whether the general path's 16-row tiles need ffn_skinny_kernel's general
+// instance: K ranges of whole steps, features of whole 16-row groups and
+// 16-byte alignment take the plain one.
+bool needs_general(const moe355_plan* p, int K, int features, int k_per_split, const void* x,
+                   const void* const* w) {
+  const int step = general_step_bytes(p) / elem_size(p->dtype);
+  if (K % step || k_per_split % step || features % 16 || !aligned16(x)) return true;
+  for (int e = 0; e < p->E; ++e)
+    if (!aligned16(w[e])) return true;
+  return false;
+}
+
+// Whether every weight row of K elements starts on a 128-byte line. Only then do
+// the general kernel's 128-byte steps fetch each line once; otherwise a line
+// serves two steps and has to stay cached in between.
+bool lines_aligned(int K, int dtype, int E, const void* const* w) {
+  if (static_cast<size_t>(K) * elem_size(dtype) % 128) return false;
+  for (int e = 0; e < E; ++e)
+    if (reinterpret_cast<uintptr_t>(w[e]) & 127) return false;
+  return true;
+}
+
+}  // namespace
+
 extern "C" {
 
 int moe355_version(void) { return 101; }
@@ -107,6 +143,17 @@ int moe355_make_plan(int T, int H, int I, int E, int K, int dtype, moe355_plan* 
 
 int moe355_make_plan_path(int T, int H, int I, int E, int K, int dtype, int path,
                           moe355_plan* p) {
+  return plan_impl(T, H, I, E, K, dtype, path, /*compact=*/false, p);
+}
+
+}  // extern "C"
+
+namespace {
+
+// The plan of moe355_make_plan_path. compact: the general path's smallest
+// workspace (64-row tiles, one K-split), for callers with a fixed scratch size.
+int plan_impl(int T, int H, int I, int E, int K, int dtype, int path, bool compact,
+              moe355_plan* p) {
   if (!p) return fail(MOE355_EINVAL, "plan is NULL");
   if (path < -1 || path > MOE355_PATH_MFMA_TILED128 || path == 3)
     return fail(MOE355_EINVAL, "unknown path %d", path);
@@ -146,7 +193,7 @@ int moe355_make_plan_path(int T, int H, int I, int E, int K, int dtype, int path
     // fine-grained 512 tokens 0.31 against 0.32), 256-row tiles above
     // (Mixtral 512 tokens: 0.67 against 0.68 ms).
     path = tiled_ok && avg > 104  ? MOE355_PATH_MFMA_TILED
-           : tiled_ok && avg > 10 ? MOE355_PATH_MFMA_TILED128
+           : tiled_ok && avg > kSkinnyRows ? MOE355_PATH_MFMA_TILED128
            : skinny_ok            ? MOE355_PATH_MFMA_SKINNY
                                   : MOE355_PATH_SIMT;
   } else if (((path == MOE355_PATH_MFMA_TILED || path == MOE355_PATH_MFMA_TILED128) &&
@@ -160,6 +207,7 @@ int moe355_make_plan_path(int T, int H, int I, int E, int K, int dtype, int path
   p->tile_rows = path == MOE355_PATH_MFMA_TILED      ? 256
                  : path == MOE355_PATH_MFMA_TILED128 ? 128
                  : path == MOE355_PATH_MFMA_SKINNY   ? 16
+                 : avg <= kSkinnyRows && !compact    ? 16
                                                      : 64;
   p->max_tiles = R > 0 ? static_cast<int>((R + static_cast<long long>(act_e) * (p->tile_rows - 1)) /
                                           p->tile_rows)
@@ -213,6 +261,20 @@ int moe355_make_plan_path(int T, int H, int I, int E, int K, int dtype, int path
     int s = 1;
     while (s < 8 && waves * s < 8192 && (I / 128) % (2 * s) == 0) s *= 2;
     p->down_splits = s;
+  } else if (!compact) {
+    // General path: the 16-row tiles as above; the 64-row ones (tiles estimated
+    // as for the tiled kernels) until there are two 128-feature items per CU,
+    // each of at least 4 steps of 128 bytes of K.
+    const bool small = p->tile_rows == 16;
+    const int nsteps = (I * esz + general_step_bytes(p) - 1) / general_step_bytes(p);
+    const long long tiles =
+        small ? p->max_tiles
+              : std::min<long long>(p->max_tiles, R / p->tile_rows + (act_e + 1) / 2);
+    const long long items = std::max(tiles, 1ll) * (small ? (H + 15) / 16 : (H + 127) / 128);
+    const long long want = small ? 8192 : 2ll * moe355::device_cu_count();
+    int s = 1;
+    while (s < 8 && items * s < want && nsteps >= (small ? 2 : 8) * s) s *= 2;
+    p->down_splits = s;
   }
 
   size_t off = 0;
@@ -234,6 +296,10 @@ int moe355_make_plan_path(int T, int H, int I, int E, int K, int dtype, int path
   p->workspace_bytes = off;
   return MOE355_OK;
 }
+
+}  // namespace
+
+extern "C" {
 
 int moe355_router_topk(const void* x, const void* gate, const float* bias, int T, int H, int E,
                        int K, int dtype, int renormalize, int round_logits, int entropy_k_min,
@@ -397,7 +463,7 @@ int permute_args(const moe355_plan* p, const void* topk_ids, int ids_int64,
   return MOE355_OK;
 }
 
-// moe355_gate_up, or with self (skinny path, <= 64 routed slots) the
+// moe355_gate_up, or with self (16-row tiles, <= 64 routed slots) the
 // self-permuting gate_up that also does the permute's work.
 int gate_up_impl(const moe355_plan* p, const void* x, const void* const* w1, int act,
                  void* workspace, void* stream, const PermuteArgs* self);
@@ -471,9 +537,18 @@ int gate_up_impl(const moe355_plan* p, const void* x, const void* const* w1, int
       a.perm = *self;
     }
     err = launch_gate_up_skinny(a, p->dtype, as_stream(stream));
+  } else if (p->tile_rows == 16) {
+    a.n_wtiles = (p->I + 15) / 16;
+    a.general = needs_general(p, p->H, p->I, p->H, x, w1);
+    if (self) {
+      a.self_permute = 1;
+      a.perm = *self;
+    }
+    err = launch_gate_up_skinny(a, p->dtype, as_stream(stream));
   } else {
-    a.n_wtiles = (p->I + 63) / 64;
-    err = launch_gate_up_simt(a, p->dtype, as_stream(stream));
+    a.tile_rows = p->tile_rows;
+    a.stream_once = lines_aligned(p->H, p->dtype, p->E, w1);
+    err = launch_gate_up_general(a, p->dtype, as_stream(stream));
   }
   return check_hip(err, "gate_up launch");
 }
@@ -495,7 +570,7 @@ int run_fused(const moe355_plan& p, const void* x, const void* const* w1, const 
               const int32_t* expert_map, int map_len, int act, void* out, int accumulate_f32,
               void* workspace, void* stream) {
   int rc;
-  if (p.path == MOE355_PATH_MFMA_SKINNY && p.rows <= 64) {
+  if (p.tile_rows == 16 && p.rows <= 64) {
     // Decode sizes (<= 64 routed slots, one wave's worth): the gate_up
     // workgroups group the routed slots themselves (one launch fewer; the
     // permute's outputs are still written for down and combine). Every
@@ -583,8 +658,20 @@ int moe355_down(const moe355_plan* p, const void* const* w2, void* workspace, vo
     a.n_wtiles = p->H / 16;
     err = launch_down_skinny(a, p->dtype, as_stream(stream));
   } else {
-    a.n_wtiles = (p->H + 63) / 64;
-    err = launch_down_simt(a, p->dtype, as_stream(stream));
+    // Splits of whole K steps; the last may be shorter (or empty: zeros).
+    const int step = general_step_bytes(p) / elem_size(p->dtype);
+    const int nsteps = (p->I + step - 1) / step;
+    a.k_per_split = (nsteps + p->down_splits - 1) / p->down_splits * step;
+    if (p->tile_rows == 16) {
+      a.n_wtiles = (p->H + 15) / 16;
+      a.general = needs_general(p, p->I, p->H, a.k_per_split, a.x, w2) ||
+                  a.k_per_split * p->down_splits != p->I;
+      err = launch_down_skinny(a, p->dtype, as_stream(stream));
+    } else {
+      a.tile_rows = p->tile_rows;
+      a.stream_once = lines_aligned(p->I, p->dtype, p->E, w2);
+      err = launch_down_general(a, p->dtype, as_stream(stream));
+    }
   }
   return check_hip(err, "down launch");
 }
@@ -636,15 +723,18 @@ int moe355_fused_experts_static(const void* x, const void* const* w1, const void
     // The tiled paths' last region holds one fp32 partial tile per CU for the
     // down projection's K-split tail; without it the down projection runs its
     // last round whole (same results up to fp32 summation order).
+    // The general path plans again without K-splits of the down projection.
     const bool tiled = p.path == MOE355_PATH_MFMA_TILED || p.path == MOE355_PATH_MFMA_TILED128;
-    if (!tiled || p.off_part > MOE355_STATIC_SCRATCH_BYTES)
+    if (p.path == MOE355_PATH_SIMT && (rc = plan_impl(T, H, I, E, K, dtype, p.path, true, &p)))
+      return rc;
+    if (p.workspace_bytes > MOE355_STATIC_SCRATCH_BYTES && (!tiled || p.off_part > MOE355_STATIC_SCRATCH_BYTES))
       return fail(MOE355_EWORKSPACE,
                   "fused_experts_static: T=%d H=%d I=%d E=%d K=%d needs %zu bytes of scratch, "
                   "more than the library's static %u bytes; use moe355_fused_experts with a "
                   "workspace",
                   T, H, I, E, K, tiled ? p.off_part : p.workspace_bytes,
                   static_cast<unsigned>(MOE355_STATIC_SCRATCH_BYTES));
-    p.workspace_bytes = p.off_part;
+    if (tiled) p.workspace_bytes = p.off_part;
   }
   void* ws = nullptr;
   if ((rc = static_scratch(stream, &ws))) return rc;

@@ -79,6 +79,19 @@ struct Vec16<f16> {
   }
 };
 
+// 16 bytes at an address of any element alignment (the general kernels take
+// such operands; gfx950 loads them in one instruction all the same).
+typedef u32x4 u32x4_any __attribute__((aligned(2)));
+
+__device__ __forceinline__ u32x4 load16_any(const void* p) {
+  return *static_cast<const u32x4_any*>(p);
+}
+
+// load16_any of data that is read once.
+__device__ __forceinline__ u32x4 load16_any_once(const void* p) {
+  return __builtin_nontemporal_load(static_cast<const u32x4_any*>(p));
+}
+
 // Pack four fp32 values into four storage elements (8 bytes for 16-bit types).
 template <typename T>
 __device__ __forceinline__ void store4(T* dst, float a, float b, float c, float d) {
@@ -238,6 +251,8 @@ struct FfnArgs {
   int y16;                 // tiled down with one K-split: y rounded to the layer dtype
   int ragged;              // full-tile kernel: per-item token-block count and rotated XCD slots
   const void* w[kMaxExperts];  // w1[e] ([2I,H]) or w2[e] ([H,I])
+  int stream_once;         // general kernel: weights of one-tile experts are read past L2
+  int general;             // skinny: sizes or alignments the aligned instances do not take
   // Skinny gate_up only, when self_permute: every workgroup groups the <= 64
   // routed slots of perm itself (no permute launch), and workgroup 0 writes
   // perm's offsets, slot_to_row, row_src and tile_map for the later stages.
@@ -281,8 +296,8 @@ hipError_t launch_gate_up_tiled(const FfnArgs& a, int dtype, hipStream_t s);
 hipError_t launch_down_tiled(const FfnArgs& a, int dtype, hipStream_t s);
 hipError_t launch_gate_up_skinny(const FfnArgs& a, int dtype, hipStream_t s);
 hipError_t launch_down_skinny(const FfnArgs& a, int dtype, hipStream_t s);
-hipError_t launch_gate_up_simt(const FfnArgs& a, int dtype, hipStream_t s);
-hipError_t launch_down_simt(const FfnArgs& a, int dtype, hipStream_t s);
+hipError_t launch_gate_up_general(const FfnArgs& a, int dtype, hipStream_t s);
+hipError_t launch_down_general(const FfnArgs& a, int dtype, hipStream_t s);
 hipError_t launch_combine(const CombineArgs& a, int out_dtype, hipStream_t s);
 // Fused residual add + RMSNorm + router (norm.hip): 16-bit types, E <= 64,
 // H a multiple of 8 up to 8192, T * E <= 8192, and E <= 16 where a logits

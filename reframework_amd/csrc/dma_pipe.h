@@ -111,6 +111,20 @@ struct Mfma16<f16> {
   }
 };
 
+// fp32 operands in the same 16-byte chunks: lane l holds chunk l / 16 of row
+// l % 16, and the i-th of the four MFMAs multiplies element i of every chunk
+// (the order of k is free as long as A and B share it).
+template <>
+struct Mfma16<float> {
+  __device__ __forceinline__ static f32x4 mma(u32x4 a, u32x4 b, f32x4 c) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      c = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a[i]), __uint_as_float(b[i]), c, 0,
+                                               0, 0);
+    return c;
+  }
+};
+
 // One work item of the persistent grouped-GEMM kernels.
 struct Tile {
   int split, wtile, e, row0, row_end;

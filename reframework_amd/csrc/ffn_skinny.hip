@@ -29,6 +29,7 @@
 #include <climits>
 
 #include "common.h"
+#include "dma_pipe.h"
 
 namespace moe355 {
 namespace {
@@ -36,35 +37,21 @@ namespace {
 constexpr int kThreads = 256;
 constexpr int kWavesPerBlock = kThreads / kWave;
 constexpr int kRows = 16;
-constexpr int kKS = 128;                 // k elements per step
-constexpr int kRowStepBytes = kKS * 2;   // 256 bytes of one row per step
+constexpr int kRowStepBytes = 256;       // bytes of one row per step
+constexpr int kStepChunks = kRowStepBytes / 16;
 constexpr int kOperandBytes = kRows * kRowStepBytes;  // 4 KB
 
-template <typename T>
-struct Mfma16;
-
-template <>
-struct Mfma16<bf16> {
-  __device__ __forceinline__ static f32x4 mma(u32x4 a, u32x4 b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
-                                                   __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-  }
-};
-
-template <>
-struct Mfma16<f16> {
-  __device__ __forceinline__ static f32x4 mma(u32x4 a, u32x4 b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a),
-                                                  __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-  }
-};
-
+// 16-byte loads of operands aligned to 16 bytes, or (kAny) to the element.
+template <bool kAny>
 __device__ __forceinline__ u32x4 load16(const void* p) {
-  return *reinterpret_cast<const u32x4*>(p);
+  if constexpr (kAny) return load16_any(p);
+  return *static_cast<const u32x4*>(p);
 }
 
+template <bool kAny>
 __device__ __forceinline__ u32x4 load16_stream(const void* p) {
-  return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
+  if constexpr (kAny) return load16_any_once(p);
+  return __builtin_nontemporal_load(static_cast<const u32x4*>(p));
 }
 
 // Grouping of <= 64 routed slots by one wave, the same stable counting sort
@@ -161,8 +148,15 @@ __device__ void group_slots(const PermuteArgs& pa, int ttile, bool write_global,
   }
 }
 
-template <typename T, bool kGateUp, bool kSelfPermute>
+// kGeneral: H, I and each split's K range are any whole number of 16-byte
+// chunks, and weights and tokens are aligned to their element only. Weight rows
+// past the last feature read the last one (their results are not stored);
+// chunks past the K range read the last one and are replaced by zeros in both
+// operands (past a weight row lies the next row, whose values may be infinite).
+template <typename T, bool kGateUp, bool kSelfPermute, bool kGeneral>
 __global__ __launch_bounds__(kThreads) void ffn_skinny_kernel(const FfnArgs a) {
+  constexpr int N = Vec16<T>::N;         // elements per 16-byte chunk
+  constexpr int kKS = kStepChunks * N;   // k elements per step
   constexpr int NOP = kGateUp ? 2 : 1;   // weight operands: gate (+ up)
   constexpr int D = kGateUp ? 2 : 4;     // steps in flight per wave
   constexpr int kSliceBytes = NOP * kOperandBytes;
@@ -193,13 +187,15 @@ __global__ __launch_bounds__(kThreads) void ffn_skinny_kernel(const FfnArgs a) {
 
   const int ld = kGateUp ? a.H : a.I;
   const int kbeg = split * a.k_per_split;
-  const int nsteps = a.k_per_split / kKS;
+  const int nchunks = kGeneral && kbeg < ld ? min(a.k_per_split, ld - kbeg) / N : 0;
+  const int nsteps = kGeneral ? (nchunks + kStepChunks - 1) / kStepChunks : a.k_per_split / kKS;
 
   // Operand o covers weight rows base(o) .. base(o)+15.
   const T* w = static_cast<const T*>(a.w[e]);
   const T* wop[NOP];
   wop[0] = w + static_cast<size_t>(group * kRows) * ld;
   if (kGateUp) wop[NOP - 1] = w + static_cast<size_t>(a.I + group * kRows) * ld;
+  const int last_row = (kGateUp ? a.I : a.H) - 1 - group * kRows;  // of this group
 
   // Load j of a step: this lane reads row 4j + lane/16, logical chunk
   // (lane%16) ^ row, so the 16 lanes of a row cover its 256 bytes.
@@ -207,7 +203,7 @@ __global__ __launch_bounds__(kThreads) void ffn_skinny_kernel(const FfnArgs a) {
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const int r = 4 * j + (lane >> 4);
-    goff[j] = static_cast<uint32_t>(r * ld + (((lane & 15) ^ r) * 8));
+    goff[j] = static_cast<uint32_t>(kGeneral ? min(r, last_row) * ld : r * ld + ((lane & 15) ^ r) * N);
   }
   // MFMA sub-step s reads row lane%16, logical chunk 4s + lane/16.
   uint32_t roff[4];
@@ -222,31 +218,60 @@ __global__ __launch_bounds__(kThreads) void ffn_skinny_kernel(const FfnArgs a) {
   const int xrow = !kGateUp     ? (valid ? prow : row0)
                    : kSelfPermute ? s_rowsrc[valid ? prow : row0]
                                   : a.row_src[valid ? prow : row0];
-  const T* xp = static_cast<const T*>(a.x) + static_cast<size_t>(xrow) * ld + (lane >> 4) * 8;
+  const T* xp = static_cast<const T*>(a.x) + static_cast<size_t>(xrow) * ld +
+                (kGeneral ? 0 : (lane >> 4) * N);
   const u32x4 zero = {0, 0, 0, 0};
 
   // Rotated walk over the K steps of this split.
   const int s0 = nsteps > 0 ? (group * 7 + split * 3) % nsteps : 0;
 
   u32x4 wr[D][NOP][4], xr[D][4];
+  auto step_at = [&](int st) {
+    const int idx = s0 + st;
+    return idx >= nsteps ? idx - nsteps : idx;
+  };
   auto issue = [&](int slot, int st) {
-    int idx = s0 + st;
-    if (idx >= nsteps) idx -= nsteps;
-    const int k = kbeg + idx * kKS;
+    const int idx = step_at(st), k = kbeg + idx * kKS;
+    if constexpr (kGeneral) {
+      const int last = nchunks - 1 - idx * kStepChunks;  // last chunk of this step in range
 #pragma unroll
-    for (int o = 0; o < NOP; ++o)
+      for (int o = 0; o < NOP; ++o)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) wr[slot][o][j] = load16_stream(wop[o] + k + goff[j]);
+        for (int j = 0; j < 4; ++j)
+          wr[slot][o][j] = load16_stream<true>(
+              wop[o] + k + goff[j] + min((lane & 15) ^ (4 * j + (lane >> 4)), last) * N);
 #pragma unroll
-    for (int s = 0; s < 4; ++s) xr[slot][s] = valid ? load16(xp + k + s * 32) : zero;
+      for (int s = 0; s < 4; ++s)
+        xr[slot][s] = load16<true>(xp + k + min(4 * s + (lane >> 4), last) * N);
+    } else {
+#pragma unroll
+      for (int o = 0; o < NOP; ++o)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) wr[slot][o][j] = load16_stream<false>(wop[o] + k + goff[j]);
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+        xr[slot][s] = valid ? load16<false>(xp + k + s * 4 * N) : zero;
+    }
   };
 
   f32x4 acc[NOP];
 #pragma unroll
   for (int o = 0; o < NOP; ++o) acc[o] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  auto consume = [&](int slot) {
+  auto consume = [&](int slot, int st) {
     uint8_t* buf = lds[wave][slot & 1];
+    if constexpr (kGeneral) {
+      const int left = nchunks - step_at(st) * kStepChunks;  // chunks of this step in range
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const bool in = ((lane & 15) ^ (4 * j + (lane >> 4))) < left;
+#pragma unroll
+        for (int o = 0; o < NOP; ++o) wr[slot][o][j] = in ? wr[slot][o][j] : zero;
+      }
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+        xr[slot][s] = valid && 4 * s + (lane >> 4) < left ? xr[slot][s] : zero;
+    }
 #pragma unroll
     for (int o = 0; o < NOP; ++o)
 #pragma unroll
@@ -260,7 +285,7 @@ __global__ __launch_bounds__(kThreads) void ffn_skinny_kernel(const FfnArgs a) {
 #pragma unroll
       for (int o = 0; o < NOP; ++o) {
         const u32x4 fa = *reinterpret_cast<const u32x4*>(buf + o * kOperandBytes + roff[s]);
-        acc[o] = Mfma16<T>::mma(fa, xr[slot][s], acc[o]);
+        acc[o] = pipe::Mfma16<T>::mma(fa, xr[slot][s], acc[o]);
       }
   };
 
@@ -271,20 +296,23 @@ __global__ __launch_bounds__(kThreads) void ffn_skinny_kernel(const FfnArgs a) {
 #pragma unroll
     for (int d = 0; d < D; ++d) {
       if (st + d < nsteps) {
-        consume(d);
+        consume(d, st + d);
         if (st + d + D < nsteps) issue(d, st + d + D);
       }
     }
   }
 
   // Lane (row, kq) holds features 4*kq + 0..3 of this 16-row group for token lane%16.
-  if (!valid) return;
+  if (!valid || (kGeneral && 4 * (lane >> 4) > last_row)) return;
   const int col = group * kRows + 4 * (lane >> 4);
   if (kGateUp) {
     const f32x4 g = acc[0], u = acc[NOP - 1];
     T* inter = static_cast<T*>(a.out) + static_cast<size_t>(prow) * a.I + col;
-    store4<T>(inter, gate_act_fast(a.act, g[0]) * u[0], gate_act_fast(a.act, g[1]) * u[1],
-              gate_act_fast(a.act, g[2]) * u[2], gate_act_fast(a.act, g[3]) * u[3]);
+    float v[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      v[r] = (std::is_same<T, float>::value ? gate_act(a.act, g[r]) : gate_act_fast(a.act, g[r])) * u[r];
+    store4<T>(inter, v[0], v[1], v[2], v[3]);
   } else {
     float* y = static_cast<float*>(a.out) + static_cast<size_t>(split) * a.R * a.H +
                static_cast<size_t>(prow) * a.H + col;
@@ -292,21 +320,33 @@ __global__ __launch_bounds__(kThreads) void ffn_skinny_kernel(const FfnArgs a) {
   }
 }
 
+template <typename T, bool kGateUp, bool kGeneral>
+void launch_skinny_tg(const FfnArgs& a, dim3 grid, hipStream_t s) {
+  if (kGateUp && a.self_permute)
+    ffn_skinny_kernel<T, kGateUp, kGateUp, kGeneral><<<grid, dim3(kThreads), 0, s>>>(a);
+  else
+    ffn_skinny_kernel<T, kGateUp, false, kGeneral><<<grid, dim3(kThreads), 0, s>>>(a);
+}
+
+template <typename T, bool kGateUp>
+void launch_skinny_t(const FfnArgs& a, dim3 grid, hipStream_t s) {
+  if (a.general)
+    launch_skinny_tg<T, kGateUp, true>(a, grid, s);
+  else
+    launch_skinny_tg<T, kGateUp, false>(a, grid, s);
+}
+
 template <bool kGateUp>
 hipError_t launch_skinny(const FfnArgs& a, int dtype, hipStream_t s) {
   if (a.n_wtiles == 0 || a.max_tiles == 0) return hipSuccess;
   if (a.self_permute && (!kGateUp || a.perm.R > kWave)) return hipErrorInvalidValue;  // one wave groups
   const dim3 grid((a.n_wtiles + kWavesPerBlock - 1) / kWavesPerBlock, a.max_tiles, a.splits);
-  if (a.self_permute) {
-    if (dtype == MOE355_BF16)
-      ffn_skinny_kernel<bf16, true, true><<<grid, dim3(kThreads), 0, s>>>(a);
-    else
-      ffn_skinny_kernel<f16, true, true><<<grid, dim3(kThreads), 0, s>>>(a);
-  } else if (dtype == MOE355_BF16) {
-    ffn_skinny_kernel<bf16, kGateUp, false><<<grid, dim3(kThreads), 0, s>>>(a);
-  } else {
-    ffn_skinny_kernel<f16, kGateUp, false><<<grid, dim3(kThreads), 0, s>>>(a);
-  }
+  if (dtype == MOE355_BF16)
+    launch_skinny_t<bf16, kGateUp>(a, grid, s);
+  else if (dtype == MOE355_F16)
+    launch_skinny_t<f16, kGateUp>(a, grid, s);
+  else
+    launch_skinny_t<float, kGateUp>(a, grid, s);
   return hipGetLastError();
 }
 

@@ -1,0 +1,135 @@
+"""The general expert-FFN path (MOE355_PATH_SIMT): fp32 layers and sizes the
+bf16/f16 tiled kernels do not take, at the edges of its tiles: 16-row tiles up
+to ten rows per expert and 64-row tiles above, K steps of 128 and 256 bytes,
+feature tiles of 16 to 128, against the fp64 oracle (the tolerances of the
+other paths' tests)."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from _helpers import DT, banner, make_bank, skewed_ids
+from oracle import oracle
+from reframework_amd import _capi
+from reframework_amd.moe import fused_experts
+from test_gpu_experts import _check, gpu_fused
+
+pytestmark = pytest.mark.gpu
+
+SIMT = _capi.PATH_SIMT
+
+
+# (H, I): smallest, below one K step, partial last steps and feature tiles of
+# either kernel, whole steps of both
+SIZES = {"f32": [(4, 4), (20, 36), (132, 68), (64, 128), (260, 324)],
+         "bf16": [(8, 8), (24, 40), (136, 200), (320, 72), (264, 520)],
+         "f16": [(8, 16), (72, 136), (392, 264)]}
+
+
+@pytest.mark.parametrize("dts,size", [(d, s) for d, ss in SIZES.items() for s in ss],
+                         ids=lambda v: str(v))
+@pytest.mark.parametrize("T", [1, 13, 20, 21, 70, 300])
+def test_general_path_sizes(dts, size, T, dev):
+    H, I = size
+    E, K = 4, 2
+    dt = DT[dts]
+    plan = _capi.make_plan(T, H, I, E, K, _capi.dtype_code(dt))
+    assert plan.path == SIMT
+    assert plan.tile_rows == (16 if T * K // min(T * K, E) <= 10 else 64)
+    banner(f"general {dts} T={T} H={H} I={I} tile={plan.tile_rows} splits={plan.down_splits}")
+    w1, w2 = make_bank(E, H, I, dt, seed=H + I)
+    x = torch.randn(T, H, generator=torch.Generator().manual_seed(T)).to(dt)
+    ids = skewed_ids(T, K, E, seed=T, skew=1.0)
+    w = np.random.default_rng(T).random((T, K)).astype(np.float32)
+    _check(gpu_fused(x, w1, w2, w, ids), x, w1, w2, w, ids)
+
+
+@pytest.mark.parametrize("dts,H,I", [("f32", 132, 260), ("bf16", 136, 200)])
+@pytest.mark.parametrize("m", [11, 16, 17, 32, 33, 48, 49, 63, 64, 65, 96, 97, 128, 129])
+def test_general_path_group_sizes(m, dts, H, I, dev):
+    # all m tokens to expert 0 plus one token on expert 3 (expert 1 and 2 empty)
+    dt = DT[dts]
+    banner(f"general {dts} group of {m}")
+    w1, w2 = make_bank(4, H, I, dt, seed=m)
+    x = torch.randn(m + 1, H, generator=torch.Generator().manual_seed(m)).to(dt)
+    ids = np.zeros((m + 1, 1), np.int64)
+    ids[-1, 0] = 3
+    w = np.ones((m + 1, 1), np.float32)
+    _check(gpu_fused(x, w1, w2, w, ids, path=SIMT), x, w1, w2, w, ids, path=SIMT)
+
+
+@pytest.mark.parametrize("T", [3, 100])
+@pytest.mark.parametrize("dts,H,I", [("f32", 132, 68), ("bf16", 136, 200), ("f16", 256, 128)])
+def test_general_path_element_alignment(dts, H, I, T, dev):
+    """Weights and tokens one element off a 16-byte boundary."""
+    dt = DT[dts]
+    E, K = 4, 2
+    banner(f"general {dts} unaligned T={T}")
+    w1, w2 = make_bank(E, H, I, dt, seed=1)
+    x = torch.randn(T, H, generator=torch.Generator().manual_seed(T)).to(dt)
+    ids = skewed_ids(T, K, E, seed=T, skew=0.5)
+    w = np.random.default_rng(T).random((T, K)).astype(np.float32)
+
+    def off(t):
+        buf = torch.empty(t.numel() + 1, dtype=dt, device=dev)
+        buf[1:] = t.reshape(-1).to(dev)
+        return buf[1:].view(t.shape)
+
+    d1, d2 = [off(t) for t in w1], [off(t) for t in w2]
+    xd, tw, ti = off(x), torch.from_numpy(w).to(dev), torch.from_numpy(ids.astype(np.int32)).to(dev)
+    plan = _capi.make_plan(T, H, I, E, K, _capi.dtype_code(dt), SIMT)
+    ws = torch.empty(plan.workspace_bytes, dtype=torch.uint8, device=dev)
+    out = torch.empty(T, H, dtype=dt, device=dev)
+    p1, p2 = [t.data_ptr() for t in d1], [t.data_ptr() for t in d2]
+    _capi.permute(plan, ti, ws)
+    _capi.gate_up(plan, xd, p1, 0, ws)
+    _capi.down(plan, p2, ws)
+    _capi.combine(plan, tw, out, False, ws)
+    _check(out, x, w1, w2, w, ids, path=SIMT)
+
+
+@pytest.mark.parametrize("T", [2, 60])
+@pytest.mark.parametrize("dts,H,I", [("f32", 132, 68), ("bf16", 136, 200)])
+def test_general_path_keeps_infinities_in_their_row(dts, H, I, T, dev):
+    """A weight row ends inside a K step and the next one is infinite: only
+    that row's feature is affected."""
+    dt = DT[dts]
+    E, K, bad = 2, 1, 17
+    w1, w2 = make_bank(E, H, I, dt, seed=5)
+    ids = np.zeros((T, K), np.int64)
+    w = np.ones((T, K), np.float32)
+    x = torch.randn(T, H, generator=torch.Generator().manual_seed(T)).to(dt)
+    ref = oracle.fused_experts(x, w1, w2, w, ids, activation=0)
+    w2[0][bad, 0] = float("inf")
+    out = fused_experts(x.to(dev), [t.to(dev) for t in w1], [t.to(dev) for t in w2],
+                        torch.from_numpy(w).to(dev), torch.from_numpy(ids).to(dev))
+    got = out.float().cpu().numpy().astype(np.float64)
+    assert not np.isfinite(got[:, bad]).any()
+    keep = np.arange(H) != bad
+    assert oracle.max_rel(got[:, keep], ref[:, keep]) <= (1e-5 if dt == torch.float32 else 2e-2)
+
+
+def test_static_scratch_drops_the_splits(dev):
+    """A call whose K-split plan needs more than the static scratch still fits
+    it without the splits, as it did before there were any."""
+    T, H, I, E, K = 500, 2048, 13056, 2, 2
+    plan = _capi.make_plan(T, H, I, E, K, _capi.F32)
+    unsplit = plan.off_y + T * K * H * 4
+    assert plan.down_splits > 1
+    assert unsplit < _capi.STATIC_SCRATCH_BYTES < plan.workspace_bytes
+    g = torch.Generator(device=dev).manual_seed(0)
+    w1 = torch.empty(E, 2 * I, H, device=dev).normal_(0, 0.02, generator=g)
+    w2 = torch.empty(E, H, I, device=dev).normal_(0, 0.02, generator=g)
+    x = torch.empty(T, H, device=dev).normal_(generator=g)
+    w, ids = torch.topk(torch.softmax(torch.empty(T, E, device=dev).normal_(generator=g), -1), K)
+    want = fused_experts(x, w1, w2, w, ids)
+    out = torch.empty_like(x)
+    _capi.fused_experts_static(x, [w1[e].data_ptr() for e in range(E)],
+                               [w2[e].data_ptr() for e in range(E)], I, w.contiguous(),
+                               ids.int().contiguous(), 0, out)
+    # the same products in fp32, summed in another order
+    assert (out - want).norm() <= 1e-5 * want.norm()
+
+
