@@ -250,7 +250,7 @@ __global__ __launch_bounds__(kThreads) void ffn_skinny_kernel(const FfnArgs a) {
         for (int j = 0; j < 4; ++j) wr[slot][o][j] = load16_stream<false>(wop[o] + k + goff[j]);
 #pragma unroll
       for (int s = 0; s < 4; ++s)
-        xr[slot][s] = valid ? load16<false>(xp + k + s * 4 * N) : zero;
+        xr[slot][s] = load16<false>(xp + k + s * 4 * N);
     }
   };
 
@@ -270,7 +270,7 @@ __global__ __launch_bounds__(kThreads) void ffn_skinny_kernel(const FfnArgs a) {
       }
 #pragma unroll
       for (int s = 0; s < 4; ++s)
-        xr[slot][s] = valid && 4 * s + (lane >> 4) < left ? xr[slot][s] : zero;
+        xr[slot][s] = 4 * s + (lane >> 4) < left ? xr[slot][s] : zero;
     }
 #pragma unroll
     for (int o = 0; o < NOP; ++o)
@@ -289,10 +289,31 @@ __global__ __launch_bounds__(kThreads) void ffn_skinny_kernel(const FfnArgs a) {
       }
   };
 
+  // While at least 2 D steps are left every issue is unconditional, so the
+  // compiler counts the loads in flight exactly and each step waits for its own
+  // loads only; under a condition it waits for all of them (experts of the
+  // Mixtral shape, 1 token: 114.8 -> 113.3 us; 8 of 66 experts of H 2048, I 1408,
+  // 1 token: 33.6 -> 30.6 us; fp32 H 1024, I 2816, 4 tokens: 48.1 -> 44.7 us).
+  // The last steps (and K ranges shorter than 2 D steps) are not worth a copy
+  // per count.
+  int st = 0;
+  if (nsteps >= 2 * D) {
 #pragma unroll
-  for (int d = 0; d < D; ++d)
-    if (d < nsteps) issue(d, d);
-  for (int st = 0; st < nsteps; st += D) {
+    for (int d = 0; d < D; ++d) issue(d, d);
+    do {
+#pragma unroll
+      for (int d = 0; d < D; ++d) {
+        consume(d, st + d);
+        issue(d, st + d + D);
+      }
+      st += D;
+    } while (st + 2 * D <= nsteps);
+  } else {
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+      if (d < nsteps) issue(d, d);
+  }
+  for (; st < nsteps; st += D) {
 #pragma unroll
     for (int d = 0; d < D; ++d) {
       if (st + d < nsteps) {
