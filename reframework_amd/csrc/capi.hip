@@ -39,6 +39,11 @@ constexpr int kMaxDevices = 64;
 
 // Average rows per active expert up to which 16-row weight-streaming tiles run.
 constexpr int kSkinnyRows = 10;
+// And up to which 128-row tile maps run the general kernel rather than the
+// persistent 128-row one (mid_sized): at 62 to 66 rows 16 experts of I 6400 gain
+// 2 % and fine-grained experts lose 1 %, at 75 the Mixtral shape gains 5 %,
+// I 6400 loses 1 %; at 94 to 100 rows 2 to 10 % are lost.
+constexpr int kMidRows = 64;
 
 size_t align256(size_t v) { return (v + 255) & ~static_cast<size_t>(255); }
 
@@ -117,6 +122,13 @@ bool needs_general(const moe355_plan* p, int K, int features, int k_per_split, c
   for (int e = 0; e < p->E; ++e)
     if (!aligned16(w[e])) return true;
   return false;
+}
+
+// Whether a 128-row tile map runs the general kernel's 128-row instance rather
+// than the persistent 128-row kernel.
+bool mid_sized(const moe355_plan* p) {
+  const long long act = std::min<long long>(p->E, p->rows);
+  return p->path == MOE355_PATH_MFMA_TILED128 && p->rows <= kMidRows * act;
 }
 
 // Whether every weight row of K elements starts on a 128-byte line. Only then do
@@ -227,7 +239,10 @@ int plan_impl(int T, int H, int I, int E, int K, int dtype, int path, bool compa
     // 128 and 256 tokens on 128-row tiles: 8): max_tiles is a worst case, and
     // sizing the split by it cut layers finer than their real tile count pays
     // for (Mixtral 256, 512 and 1024 tokens: down 0.201, 0.225 and 0.318 ms
-    // with the worst case, 0.183, 0.204 and 0.283 with the estimate).
+    // with the worst case, 0.183, 0.204 and 0.283 with the estimate). The general
+    // kernel takes the same splits on these maps (down + combine on the Mixtral
+    // shape at 197 tokens: 170 us with one, 171 with these 2, 188 with 4); one
+    // split where this picks more would round y to 16 bits.
     const double est_tiles =
         std::min(static_cast<double>(p->max_tiles),
                  act_e * std::max(1.0, static_cast<double>(R) / act_e / p->tile_rows + 0.5));
@@ -262,16 +277,20 @@ int plan_impl(int T, int H, int I, int E, int K, int dtype, int path, bool compa
     while (s < 8 && waves * s < 8192 && (I / 128) % (2 * s) == 0) s *= 2;
     p->down_splits = s;
   } else if (!compact) {
-    // General path: the 16-row tiles as above; the 64-row ones (tiles estimated
-    // as for the tiled kernels) until there are two 128-feature items per CU,
-    // each of at least 4 steps of 128 bytes of K.
+    // General path: the 16-row tiles as above; the 64-row ones by items of 128
+    // features, each of at least 4 steps of 128 bytes of K: 16-bit types while
+    // they leave a quarter of the CUs idle (H 1240, I 3304, 12 experts, 333 tokens: down +
+    // combine 49 us with one split, 51 with 2, 54 with 4), fp32, bound by its
+    // MFMAs, up to two per CU (H 1024, I 2816, 512 tokens: 116, 90, 87 and 84 us
+    // with 1, 2, 4 and 8).
     const bool small = p->tile_rows == 16;
     const int nsteps = (I * esz + general_step_bytes(p) - 1) / general_step_bytes(p);
     const long long tiles =
         small ? p->max_tiles
               : std::min<long long>(p->max_tiles, R / p->tile_rows + (act_e + 1) / 2);
     const long long items = std::max(tiles, 1ll) * (small ? (H + 15) / 16 : (H + 127) / 128);
-    const long long want = small ? 8192 : 2ll * moe355::device_cu_count();
+    const long long cus = moe355::device_cu_count();
+    const long long want = small ? 8192 : dtype == MOE355_F32 ? 2 * cus : cus * 3 / 4;
     int s = 1;
     while (s < 8 && items * s < want && nsteps >= (small ? 2 : 8) * s) s *= 2;
     p->down_splits = s;
@@ -520,7 +539,11 @@ int gate_up_impl(const moe355_plan* p, const void* x, const void* const* w1, int
   a.splits = 1; a.k_per_split = p->H; a.act = act;
   for (int e = 0; e < p->E; ++e) a.w[e] = w1[e];
   hipError_t err;
-  if (p->path == MOE355_PATH_MFMA_TILED || p->path == MOE355_PATH_MFMA_TILED128) {
+  if (mid_sized(p)) {
+    a.tile_rows = p->tile_rows;
+    a.stream_once = lines_aligned(p->H, p->dtype, p->E, w1);
+    err = launch_gate_up_general(a, p->dtype, as_stream(stream));
+  } else if (p->path == MOE355_PATH_MFMA_TILED || p->path == MOE355_PATH_MFMA_TILED128) {
     a.n_wtiles = p->I / 128;
     a.tile_rows = p->tile_rows;
     a.ragged = ragged_tiles(p);
@@ -643,7 +666,12 @@ int moe355_down(const moe355_plan* p, const void* const* w2, void* workspace, vo
   a.splits = p->down_splits; a.k_per_split = p->I / p->down_splits; a.act = 0;
   for (int e = 0; e < p->E; ++e) a.w[e] = w2[e];
   hipError_t err;
-  if (p->path == MOE355_PATH_MFMA_TILED || p->path == MOE355_PATH_MFMA_TILED128) {
+  if (mid_sized(p)) {
+    a.tile_rows = p->tile_rows;
+    a.y16 = y_narrow(p);
+    a.stream_once = lines_aligned(p->I, p->dtype, p->E, w2);
+    err = launch_down_general(a, p->dtype, as_stream(stream));
+  } else if (p->path == MOE355_PATH_MFMA_TILED || p->path == MOE355_PATH_MFMA_TILED128) {
     a.n_wtiles = p->H / 256;
     a.tile_rows = p->tile_rows;
     a.ragged = ragged_tiles(p);

@@ -1,8 +1,8 @@
 // Grouped expert FFN on one workgroup per (K-split, weight tile, token tile)
-// item: fp32 layers, and sizes the bf16/f16 tiled kernels do not take (H no
-// multiple of 256, I no multiple of 128, token rows past 2 GB). Any H and I of
-// whole 16-byte vectors run here. Groups of up to ten rows run
-// ffn_skinny_kernel's general instances instead.
+// item: fp32 layers, sizes the bf16/f16 tiled kernels do not take (H no multiple
+// of 256, I no multiple of 128, token rows past 2 GB), and bf16/f16 groups of
+// about 10 to 64 rows on 128-row token tiles. Any H and I of whole 16-byte
+// vectors run here. Groups of up to ten rows run ffn_skinny_kernel instead.
 //
 // Replaces the per-expert GEMMs of fused_experts (reframework/moe/fused.py:76-83)
 // with the same contract as the tiled kernels: items over the permute's tile
@@ -31,7 +31,16 @@
 // element per LDS read (gate_up + down, 64 x 64 tiles, 16 k a step). Layers,
 // before -> now: fp32 H 1024, I 2816, 8 experts top-2, 512 tokens 1.04 -> 0.21 ms
 // (86 TFLOP/s), 128 tokens 0.88 -> 0.10 ms; bf16 H 1240, I 3304, 12 experts
-// top-3, 333 tokens 1.44 -> 0.13 ms, 60 tokens 1.27 -> 0.088 ms.
+// top-3, 333 tokens 1.44 -> 0.126 ms, 60 tokens 1.27 -> 0.085 ms.
+//
+// Groups of 10 to 64 rows of the tiled sizes are bound by the weight stream.
+// Against the persistent 128-row kernel (one workgroup per CU, which overlaps
+// nothing with its barriers and epilogues and shares L2 between weights and
+// tokens), layers: Mixtral shape, 44 / 197 / 256 tokens 559 / 567 / 577 ->
+// 450 / 498 / 521 us; 16 experts of I 6400, 300 tokens 486 -> 444; 66 experts
+// top-8 of H 2048, I 1408, 128 / 300 tokens 249 / 256 -> 219 / 237. At about 75
+// rows per expert both take the same time, and above the persistent kernel
+// wins (mid_sized in capi.hip).
 #include "common.h"
 #include "dma_pipe.h"
 
@@ -254,9 +263,12 @@ __global__ __launch_bounds__(kThreads, 2) void ffn_general_kernel(const FfnArgs 
 // Tiles measured at the layers above (us): fp32 64 x 64 one step deep 205 at 512
 // tokens, two steps deep 211, 128 x 64 two deep 263; bf16 128 x 64 two steps deep
 // 129-131, 64 x 64 145-148, and with weights loaded past L2 206 (rows there
-// do not start on 128-byte lines, so every line serves two steps).
+// do not start on 128-byte lines, so every line serves two steps). Mixtral shape
+// on 128-row maps, 100 and 197 tokens: 128 x 128 two deep 467 and 488, one deep
+// 484 and 525, 64 x 128 one deep 476 and 544, 256 x 64 (64-row maps) 500 and 507.
 typedef Config<64, 64, 1> ConfigF32;
 typedef Config<128, 64, 2> Config16;
+typedef Config<128, 128, 2> ConfigMid;
 
 template <typename T, bool kGateUp, typename C>
 hipError_t launch_items(FfnArgs a, hipStream_t s) {
@@ -271,6 +283,9 @@ hipError_t launch_items(FfnArgs a, hipStream_t s) {
 
 template <bool kGateUp>
 hipError_t launch_general(const FfnArgs& a, int dtype, hipStream_t s) {
+  if (a.tile_rows == 128 && dtype != MOE355_F32)
+    return dtype == MOE355_BF16 ? launch_items<bf16, kGateUp, ConfigMid>(a, s)
+                                : launch_items<f16, kGateUp, ConfigMid>(a, s);
   if (dtype == MOE355_BF16) return launch_items<bf16, kGateUp, Config16>(a, s);
   if (dtype == MOE355_F16) return launch_items<f16, kGateUp, Config16>(a, s);
   return launch_items<float, kGateUp, ConfigF32>(a, s);

@@ -60,6 +60,25 @@ def test_general_path_group_sizes(m, dts, H, I, dev):
     _check(gpu_fused(x, w1, w2, w, ids, path=SIMT), x, w1, w2, w, ids, path=SIMT)
 
 
+@pytest.mark.parametrize("m", [31, 33, 96, 97, 128, 129, 191, 193])
+@pytest.mark.parametrize("dts,I", [("bf16", 128), ("f16", 640)])
+def test_128_row_maps_up_to_64_rows_per_expert(dts, I, m, dev):
+    # one large group among three experts: its tile(s) of every 32-row count, y
+    # rounded (one K-split) or in fp32 planes; past 64 rows on average the
+    # persistent 128-row kernel runs the same plan
+    H, E, T = 256, 3, m + 2
+    dt = DT[dts]
+    plan = _capi.make_plan(T, H, I, E, 1, _capi.dtype_code(dt), _capi.PATH_MFMA_TILED128)
+    banner(f"128-row map {dts} I={I} group of {m} splits={plan.down_splits}")
+    w1, w2 = make_bank(E, H, I, dt, seed=m)
+    x = torch.randn(T, H, generator=torch.Generator().manual_seed(m)).to(dt)
+    ids = np.full((T, 1), 1, np.int64)
+    ids[0, 0], ids[-1, 0] = 2, 0
+    w = np.ones((T, 1), np.float32)
+    path = _capi.PATH_MFMA_TILED128
+    _check(gpu_fused(x, w1, w2, w, ids, path=path), x, w1, w2, w, ids, path=path)
+
+
 @pytest.mark.parametrize("T", [3, 100])
 @pytest.mark.parametrize("dts,H,I", [("f32", 132, 68), ("bf16", 136, 200), ("f16", 256, 128)])
 def test_general_path_element_alignment(dts, H, I, T, dev):
