@@ -190,8 +190,15 @@ def act_code(activation: str) -> int:
 
 
 def stream_handle(device: torch.device, stream: Optional[torch.cuda.Stream] = None) -> int:
-    s = stream if stream is not None else torch.cuda.current_stream(device)
-    return int(s.cuda_stream)
+    """Raw handle of ``stream``, or of the current stream of ``device``. The
+    latter is asked for directly: building a Stream object for it takes about
+    4 us of host time, and a forward asks three times (H 1024, 4 tokens: 43 us
+    of host time with Stream objects, the kernels 30)."""
+    if stream is not None:
+        return int(stream.cuda_stream)
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None
+                                              else index)
 
 
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
