@@ -195,8 +195,6 @@ __global__ __launch_bounds__(kThreads) void add_rmsnorm_router_kernel(const Norm
   __shared__ float red[TB][kWaves];
   __shared__ float part[kWaves][64];
   __shared__ float lg[TB][kMaxRouterExperts];
-  __shared__ float psel[kWaves][kMaxRouterExperts];
-  __shared__ int32_t isel[kWaves][kMaxRouterExperts];
 
   u32x4 npk[TB][CPT];  // the rows: residual sums, then normed, rounded to T
   u32x4 gcur[PF ? CPT : 1][PF ? EG : 1];  // this pass's gate chunks
@@ -359,7 +357,7 @@ __global__ __launch_bounds__(kThreads) void add_rmsnorm_router_kernel(const Norm
     }
   }
   for (int t = wave; t < ntok; t += kWaves)
-    wave_topk(lg[t], ra.E, ra.K, ra.renormalize, 0, psel[wave], isel[wave],
+    wave_topk(lg[t], ra.E, ra.K, ra.renormalize, 0,
               ra.topk_w + static_cast<size_t>(t0 + t) * ra.out_ld,
               ra.topk_ids + static_cast<size_t>(t0 + t) * ra.out_ld, lane);
 }

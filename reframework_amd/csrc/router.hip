@@ -29,8 +29,6 @@ __global__ __launch_bounds__(kThreads) void router_kernel(const RouterArgs a) {
   constexpr int SH = 6 - log2i(NV);      // lane bits below the value index
   __shared__ float part[kThreads / kWave][64];
   __shared__ float lg[TB][kMaxExperts];
-  __shared__ float psel[kThreads / kWave][kMaxExperts];
-  __shared__ int32_t isel[kThreads / kWave][kMaxExperts];
 
   const int t0 = blockIdx.x * TB;
   const int ntok = min(TB, a.T - t0);
@@ -95,7 +93,7 @@ __global__ __launch_bounds__(kThreads) void router_kernel(const RouterArgs a) {
   }
 
   for (int t = wave; t < ntok; t += kThreads / kWave)
-    wave_topk(lg[t], a.E, a.K, a.renormalize, a.entropy_k_min, psel[wave], isel[wave],
+    wave_topk(lg[t], a.E, a.K, a.renormalize, a.entropy_k_min,
               a.topk_w + static_cast<size_t>(t0 + t) * a.out_ld,
               a.topk_ids + static_cast<size_t>(t0 + t) * a.out_ld, lane);
 }
@@ -297,13 +295,10 @@ __global__ __launch_bounds__(kThreads) void router_logits_kernel(const RouterArg
 // One wave per token on given fp32 logits (logits_in, or the logits_out the
 // split router just wrote); results at row t of [T, out_ld] arrays.
 __global__ __launch_bounds__(kThreads) void topk_logits_kernel(const RouterArgs a) {
-  __shared__ float psel[kThreads / kWave][kMaxExperts];
-  __shared__ int32_t isel[kThreads / kWave][kMaxExperts];
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
   const int t = blockIdx.x * (kThreads / kWave) + wave;
   if (t >= a.T) return;
-  wave_topk(a.logits_in + static_cast<size_t>(t) * a.E, a.E, a.K, a.renormalize,
-            a.entropy_k_min, psel[wave], isel[wave],
+  wave_topk(a.logits_in + static_cast<size_t>(t) * a.E, a.E, a.K, a.renormalize, a.entropy_k_min,
             a.topk_w + static_cast<size_t>(t) * a.out_ld,
             a.topk_ids + static_cast<size_t>(t) * a.out_ld, lane);
 }

@@ -150,5 +150,3 @@ def test_static_scratch_drops_the_splits(dev):
                                ids.int().contiguous(), 0, out)
     # the same products in fp32, summed in another order
     assert (out - want).norm() <= 1e-5 * want.norm()
-
-
