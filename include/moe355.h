@@ -172,8 +172,8 @@ int moe355_topk_from_logits(const float* logits, int T, int E, int K, int renorm
  * current device's CU count (256 without a device) to choose the down
  * projection's K-split, and launches nothing. The kernel family follows the
  * average rows per active expert (T*K / min(T*K, E)): up to 10 skinny, up to
- * 104 the tiled kernel on 128-row tiles, above it 256-row tiles; fp32 and
- * sizes these kernels do not take run MOE355_PATH_SIMT, on 16-row tiles up to
+ * 104 128-row token tiles, above it 256-row tiles; fp32 and sizes that the
+ * family of their group size does not take run MOE355_PATH_SIMT, on 16-row tiles up to
  * 10 rows and 64-row tiles above. */
 int moe355_make_plan(int T, int H, int I, int E, int K, int dtype, moe355_plan* plan);
 

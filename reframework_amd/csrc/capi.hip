@@ -204,10 +204,14 @@ int plan_impl(int T, int H, int I, int E, int K, int dtype, int path, bool compa
     // tokens: 0.55 and 0.59 ms against 0.56 and 0.65 with 256-row tiles;
     // fine-grained 512 tokens 0.31 against 0.32), 256-row tiles above
     // (Mixtral 512 tokens: 0.67 against 0.68 ms).
-    path = tiled_ok && avg > 104  ? MOE355_PATH_MFMA_TILED
-           : tiled_ok && avg > kSkinnyRows ? MOE355_PATH_MFMA_TILED128
-           : skinny_ok            ? MOE355_PATH_MFMA_SKINNY
-                                  : MOE355_PATH_SIMT;
+    // Sizes only the weight-streaming kernel tiles (H a multiple of 128 but not
+    // of 256, or tokens past 2 GB) leave it for the general kernel at the same 10
+    // rows (H 1152, I 3200, 8 experts top-2, 48 / 128 / 333 tokens: 53 / 97 / 198 us
+    // streaming, 48 / 53 / 78 general).
+    path = tiled_ok && avg > 104                  ? MOE355_PATH_MFMA_TILED
+           : tiled_ok && avg > kSkinnyRows        ? MOE355_PATH_MFMA_TILED128
+           : skinny_ok && avg <= kSkinnyRows      ? MOE355_PATH_MFMA_SKINNY
+                                                  : MOE355_PATH_SIMT;
   } else if (((path == MOE355_PATH_MFMA_TILED || path == MOE355_PATH_MFMA_TILED128) &&
               !tiled_ok) ||
              (path == MOE355_PATH_MFMA_SKINNY && !skinny_ok)) {

@@ -60,6 +60,21 @@ def test_general_path_group_sizes(m, dts, H, I, dev):
     _check(gpu_fused(x, w1, w2, w, ids, path=SIMT), x, w1, w2, w, ids, path=SIMT)
 
 
+@pytest.mark.parametrize("T,path,tile", [(40, _capi.PATH_MFMA_SKINNY, 16), (44, SIMT, 64),
+                                         (300, SIMT, 64)])
+def test_sizes_only_the_streaming_kernel_tiles(T, path, tile, dev):
+    # H a multiple of 128, not of 256: weight streaming up to 10 rows per expert
+    H, I, E, K = 384, 256, 4, 1
+    plan = _capi.make_plan(T, H, I, E, K, _capi.BF16)
+    assert (plan.path, plan.tile_rows) == (path, tile)
+    banner(f"H={H} T={T} path={path}")
+    w1, w2 = make_bank(E, H, I, torch.bfloat16, seed=T)
+    x = torch.randn(T, H, generator=torch.Generator().manual_seed(T)).to(torch.bfloat16)
+    ids = skewed_ids(T, K, E, seed=T, skew=0.5)
+    w = np.random.default_rng(T).random((T, K)).astype(np.float32)
+    _check(gpu_fused(x, w1, w2, w, ids), x, w1, w2, w, ids)
+
+
 @pytest.mark.parametrize("m", [31, 33, 96, 97, 128, 129, 191, 193])
 @pytest.mark.parametrize("dts,I", [("bf16", 128), ("f16", 640)])
 def test_128_row_maps_up_to_64_rows_per_expert(dts, I, m, dev):

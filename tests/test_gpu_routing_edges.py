@@ -23,7 +23,7 @@ def test_topk_past_one_per_lane(E, K, dev):
     rng = np.random.default_rng(E + K)
     logits = (rng.normal(size=(37, E)) * 2).astype(np.float32)
     logits[::3] = np.round(logits[::3])      # exact ties
-    logits[1::5, E // 2:] = -np.inf          # masked experts, selected last in id order
+    logits[1::5, (E + 1) // 2:] = -np.inf    # masked experts, selected last in id order
     for renorm in (True, False):
         w, ids = torch_fused_topk(torch.from_numpy(logits).to(dev), K, renorm)
         ow, oids = oracle.topk(logits, K, renorm)
