@@ -57,7 +57,7 @@ extern "C" {
 #define MOE355_PATH_SIMT 2        /* fp32 layers and sizes the other families do not take: MFMA tiles
                                      (fp32 MFMA for fp32) of 16 or 64 token rows */
 /* 3 is unused (a 256x64-tile family that no workload chose was removed) */
-#define MOE355_PATH_MFMA_TILED128 4 /* the 256x256 kernel on 128-row token tiles, groups of ~128 rows */
+#define MOE355_PATH_MFMA_TILED128 4 /* 128-row token tiles, groups of ~10 to 104 rows */
 
 /* Execution plan of one fused_experts call. Filled by moe355_make_plan() from
  * the shape alone (no device data), so every stage sees the same layout. */

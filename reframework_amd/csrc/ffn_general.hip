@@ -25,19 +25,20 @@
 // may be infinite) and operands need not be 16-byte aligned.
 //
 // fp32 is bound by its MFMA rate (157 TFLOP/s, a sixteenth of bf16's; an
-// all-register probe holds 150) and by the last round of items, which is why
-// its tile is small. 16-bit sizes on this path are bound by the weight stream
+// all-register probe holds 150; the MFMAs are busy 73 to 80 % of the cycles in
+// which a CU holds work) and by the last round of items, which is why its tile
+// is small. 16-bit sizes on this path are bound by the weight stream
 // and the LDS. Before, one kernel did both with fp32 FMAs on the VALU, one
 // element per LDS read (gate_up + down, 64 x 64 tiles, 16 k a step). Layers,
 // before -> now: fp32 H 1024, I 2816, 8 experts top-2, 512 tokens 1.04 -> 0.21 ms
 // (86 TFLOP/s), 128 tokens 0.88 -> 0.10 ms; bf16 H 1240, I 3304, 12 experts
-// top-3, 333 tokens 1.44 -> 0.126 ms, 60 tokens 1.27 -> 0.085 ms.
+// top-3, 333 tokens 1.44 -> 0.121 ms, 60 tokens 1.27 -> 0.085 ms.
 //
 // Groups of 10 to 64 rows of the tiled sizes are bound by the weight stream.
 // Against the persistent 128-row kernel (one workgroup per CU, which overlaps
 // nothing with its barriers and epilogues and shares L2 between weights and
 // tokens), layers: Mixtral shape, 44 / 197 / 256 tokens 559 / 567 / 577 ->
-// 450 / 498 / 521 us; 16 experts of I 6400, 300 tokens 486 -> 444; 66 experts
+// 450 / 479 / 513 us; 16 experts of I 6400, 300 tokens 486 -> 444; 66 experts
 // top-8 of H 2048, I 1408, 128 / 300 tokens 249 / 256 -> 219 / 237. At about 75
 // rows per expert both take the same time, and above the persistent kernel
 // wins (mid_sized in capi.hip).

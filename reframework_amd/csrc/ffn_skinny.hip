@@ -1,7 +1,7 @@
 // Grouped expert FFN for decode-sized groups (a few tokens per expert).
 //
 // Replaces the same per-expert GEMMs as the tiled kernel
-// (reframework/moe/fused.py:76-83) when each expert sees <= ~32 rows. Then the
+// (reframework/moe/fused.py:76-83) up to about 10 rows per expert. Then the
 // layer is a weight stream: every routed expert's 3*H*I weights are read once
 // and meet only a handful of tokens, so the kernel is built for HBM bandwidth.
 //
@@ -26,6 +26,9 @@
 // reads what it wrote. gate_up fuses the gated activation; down writes fp32
 // partials per K-split, which the combine kernel sums, so the short down
 // projection of a decode step still spreads over every CU.
+//
+// fp32 layers run it too (pipe::Mfma16<float>), and the general instances take
+// any H and I of whole 16-byte vectors and operands of any element alignment.
 #include <climits>
 
 #include "common.h"
