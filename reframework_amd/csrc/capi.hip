@@ -567,6 +567,7 @@ int gate_up_impl(const moe355_plan* p, const void* x, const void* const* w1, int
   } else if (p->tile_rows == 16) {
     a.n_wtiles = (p->I + 15) / 16;
     a.general = needs_general(p, p->H, p->I, p->H, x, w1);
+    a.exact_act = 1;
     if (self) {
       a.self_permute = 1;
       a.perm = *self;

@@ -138,11 +138,12 @@ __device__ __forceinline__ float sigmoid_hw(float z) {
   return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(z * -1.4426950408889634f));
 }
 
-// gate_act for the 16-bit (bf16/f16) kernels, whose outputs are rounded to 8
-// or 11 significant bits: the relative error of sigmoid_hw (~3e-7) is far below
-// that rounding, and the precise expf and IEEE division of gate_act cost about
-// 30 VALU instructions per element in an epilogue that keeps the MFMA pipe
-// idle. silu(g) = g * sigmoid(g); gelu_tanh(g) = g/2 * (1 + tanh(u)) =
+// gate_act for the 16-bit (bf16/f16) tiled and weight-streaming families, whose
+// outputs are rounded to 8 or 11 significant bits: the relative error of
+// sigmoid_hw (~3e-7) is far below that rounding, and the precise expf and IEEE
+// division of gate_act cost about 30 VALU instructions per element in an
+// epilogue that keeps the MFMA pipe idle. MOE355_PATH_SIMT applies gate_act in
+// every type. silu(g) = g * sigmoid(g); gelu_tanh(g) = g/2 * (1 + tanh(u)) =
 // g * sigmoid(2u) with u = sqrt(2/pi) * (g + 0.044715 g^3); erf-gelu keeps erff.
 __device__ __forceinline__ float gate_act_fast(int act, float g) {
   if (act == MOE355_ACT_SILU) return g * sigmoid_hw(g);
@@ -253,6 +254,7 @@ struct FfnArgs {
   const void* w[kMaxExperts];  // w1[e] ([2I,H]) or w2[e] ([H,I])
   int stream_once;         // general kernel: weights of one-tile experts are read past L2
   int general;             // skinny: sizes or alignments the aligned instances do not take
+  int exact_act;           // skinny gate_up: gate_act for 16-bit types too (MOE355_PATH_SIMT)
   // Skinny gate_up only, when self_permute: every workgroup groups the <= 64
   // routed slots of perm itself (no permute launch), and workgroup 0 writes
   // perm's offsets, slot_to_row, row_src and tile_map for the later stages.

@@ -53,9 +53,12 @@ constexpr int kRowBytes = 128;  // bytes of one operand row per step
 constexpr int kChunks = kRowBytes / 16;
 constexpr int kRowsPerPass = kThreads / kChunks;  // 32 rows per load of the workgroup
 
-template <int W, int T, int Depth>
+// kFastAct: gate_act_fast, on the plans that the tiled kernels share (128-row
+// maps); MOE355_PATH_SIMT applies gate_act in every type.
+template <int W, int T, int Depth, bool FastAct = false>
 struct Config {
   static constexpr int kW = W, kT = T, kDepth = Depth;
+  static constexpr bool kFastAct = FastAct;
 };
 
 // LDS place of chunk c of row r: 16 rows read at one chunk hit 16 distinct
@@ -257,7 +260,7 @@ __global__ __launch_bounds__(kThreads, 2) void ffn_general_kernel(const FfnArgs 
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const float g = acc[i][j][r], u = acc[i + NI / 2][j][r];
-          v[r] = (std::is_same<T, float>::value ? gate_act(a.act, g) : gate_act_fast(a.act, g)) * u;
+          v[r] = (C::kFastAct ? gate_act_fast(a.act, g) : gate_act(a.act, g)) * u;
         }
         store4<T>(static_cast<T*>(a.out) + static_cast<size_t>(prow) * a.I + f, v[0], v[1], v[2],
                   v[3]);
@@ -286,7 +289,7 @@ __global__ __launch_bounds__(kThreads, 2) void ffn_general_kernel(const FfnArgs 
 // 484 and 525, 64 x 128 one deep 476 and 544, 256 x 64 (64-row maps) 500 and 507.
 typedef Config<64, 64, 1> ConfigF32;
 typedef Config<128, 64, 2> Config16;
-typedef Config<128, 128, 2> ConfigMid;
+typedef Config<128, 128, 2, true> ConfigMid;
 
 template <typename T, bool kGateUp, typename C>
 hipError_t launch_items(FfnArgs a, hipStream_t s) {

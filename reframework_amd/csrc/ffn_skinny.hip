@@ -333,9 +333,14 @@ __global__ __launch_bounds__(kThreads) void ffn_skinny_kernel(const FfnArgs a) {
     const f32x4 g = acc[0], u = acc[NOP - 1];
     T* inter = static_cast<T*>(a.out) + static_cast<size_t>(prow) * a.I + col;
     float v[4];
+    // fp32 and the general instances run on MOE355_PATH_SIMT only.
+    if (std::is_same<T, float>::value || kGeneral || a.exact_act) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
-      v[r] = (std::is_same<T, float>::value ? gate_act(a.act, g[r]) : gate_act_fast(a.act, g[r])) * u[r];
+      for (int r = 0; r < 4; ++r) v[r] = gate_act(a.act, g[r]) * u[r];
+    } else {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = gate_act_fast(a.act, g[r]) * u[r];
+    }
     store4<T>(inter, v[0], v[1], v[2], v[3]);
   } else {
     float* y = static_cast<float*>(a.out) + static_cast<size_t>(split) * a.R * a.H +

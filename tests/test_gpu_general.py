@@ -145,6 +145,29 @@ def test_general_path_keeps_infinities_in_their_row(dts, H, I, T, dev):
     assert oracle.max_rel(got[:, keep], ref[:, keep]) <= (1e-5 if dt == torch.float32 else 2e-2)
 
 
+@pytest.mark.parametrize("T,H,I", [(3, 136, 200), (3, 256, 144), (60, 136, 200)],
+                         ids=["streaming general", "streaming plain", "64-row tiles"])
+def test_general_path_applies_the_full_precision_activation(T, H, I, dev):
+    """SiLU at -88.5 .. -87.5 is about -5e-37: 1 / (1 + e^88) lies below the
+    smallest normal fp32 number, which the hardware reciprocal of the other
+    families flushes to zero and the fp32 division of this path does not."""
+    banner(f"general activation T={T} H={H} I={I}")
+    E, dt = 2, torch.bfloat16
+    assert _capi.make_plan(T, H, I, E, 1, _capi.BF16).path == SIMT
+    g = -87.5 - 0.5 * (torch.arange(I) % 3)              # exact in bf16
+    x, w1 = torch.zeros(T, H), torch.zeros(2 * I, H)
+    x[:, 0], w1[:I, 0], w1[I:, 0] = 1.0, g, 1.0          # gate g, up 1, both exact
+    w2 = torch.zeros(H, I)
+    n = min(H, I)
+    w2[range(n), range(n)] = 1.0                         # output h is the intermediate h
+    ids = np.arange(T)[:, None] % E
+    out = gpu_fused(x.to(dt), [w1.to(dt)] * E, [w2.to(dt)] * E, np.ones((T, 1), np.float32), ids)
+    want = (g.double() / (1.0 + torch.exp(-g.double())))[:n].numpy()
+    got = out.double().cpu().numpy()[:, :n]
+    # the intermediate is rounded to bf16 once: 2^-8 of the value, a little for expf
+    assert np.max(np.abs(got - want) / np.abs(want)) <= 2.0 ** -8 * 1.01
+
+
 def test_static_scratch_drops_the_splits(dev):
     """A call whose K-split plan needs more than the static scratch still fits
     it without the splits, as it did before there were any."""
