@@ -190,15 +190,17 @@ def act_code(activation: str) -> int:
 
 
 def stream_handle(device: torch.device, stream: Optional[torch.cuda.Stream] = None) -> int:
-    """Raw handle of ``stream``, or of the current stream of ``device``. The
-    latter is asked for directly: building a Stream object for it takes about
-    4 us of host time, and a forward asks three times (H 1024, 4 tokens: 43 us
-    of host time with Stream objects, the kernels 30)."""
+    """Raw handle of ``stream``, or of the current stream of ``device``. For a
+    numbered GPU the latter is asked for directly: building a Stream object for it
+    takes about 4 us of host time, and a forward asks three times (H 1024, 4
+    tokens: 43 us of host time with Stream objects, the kernels 30). Any other
+    device goes through ``torch.cuda.current_stream``, which refuses one that is
+    not a GPU: the kernels would be given host pointers."""
     if stream is not None:
         return int(stream.cuda_stream)
-    index = device.index
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None
-                                              else index)
+    if isinstance(device, torch.device) and device.type == "cuda" and device.index is not None:
+        return torch._C._cuda_getCurrentRawStream(device.index)
+    return int(torch.cuda.current_stream(device).cuda_stream)
 
 
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:

@@ -8,6 +8,7 @@ import ctypes
 
 import numpy as np
 import pytest
+import torch
 
 from reframework_amd import _capi
 
@@ -189,3 +190,25 @@ def test_activation_codes():
     assert _capi.act_code("silu") == 0 and _capi.act_code("gelu_tanh") == 2
     with pytest.raises(ValueError, match="unknown gated activation"):
         _capi.act_code("relu")
+
+
+def test_a_device_that_is_not_a_gpu_has_no_stream(monkeypatch):
+    """Also with a GPU present (here: pretended), host tensors are refused before
+    the library is given their pointers."""
+    def reached(*args):
+        raise AssertionError("the library was called")
+
+    for name in ("moe355_topk_from_logits", "moe355_cast_f32"):
+        monkeypatch.setattr(_capi.lib(), name, reached)
+    monkeypatch.setattr(torch.cuda, "_lazy_init", lambda: None)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda index: 0x1000 + index,
+                        raising=False)
+    assert _capi.stream_handle(torch.device("cuda:3")) == 0x1003
+    with pytest.raises(ValueError, match="cpu"):
+        _capi.stream_handle(torch.device("cpu"))
+    logits, w = torch.zeros(2, 8), torch.zeros(2, 2)
+    with pytest.raises(ValueError, match="cpu"):
+        _capi.topk_from_logits(logits, 2, True, w, torch.zeros(2, 2, dtype=torch.int32))
+    with pytest.raises(ValueError, match="cpu"):
+        _capi.cast_f32(logits, torch.zeros(2, 8, dtype=torch.bfloat16))
