@@ -42,6 +42,9 @@
 // top-8 of H 2048, I 1408, 128 / 300 tokens 249 / 256 -> 219 / 237. At about 75
 // rows per expert both take the same time, and above the persistent kernel
 // wins (mid_sized in capi.hip).
+#include <algorithm>
+#include <climits>
+
 #include "common.h"
 #include "dma_pipe.h"
 
@@ -49,6 +52,7 @@ namespace moe355 {
 namespace {
 
 constexpr int kThreads = 256;
+constexpr int kGridX = 1 << 22;  // workgroups per grid row: HIP takes fewer than 2^32 threads in x
 constexpr int kRowBytes = 128;  // bytes of one operand row per step
 constexpr int kChunks = kRowBytes / 16;
 constexpr int kRowsPerPass = kThreads / kChunks;  // 32 rows per load of the workgroup
@@ -89,19 +93,20 @@ __global__ __launch_bounds__(kThreads, 2) void ffn_general_kernel(const FfnArgs 
   // gate_up 61 / 50 / 60: its few unequal items spread over the CUs).
   const int n_t = a.tile_map[0];
   const int n_q = a.n_wtiles * a.splits, n_items = n_t * n_q;
-  if (static_cast<int>(blockIdx.x) >= n_items) return;
+  const int pid = blockIdx.y * gridDim.x + blockIdx.x;  // rows of kGridX keep the XCD of pid % 8
+  if (pid >= n_items) return;
   int tt, q0;
   if (n_q % 8) {
-    const int L = xcd_remap(blockIdx.x, n_items);
+    const int L = xcd_remap(pid, n_items);
     tt = L % n_t;
     q0 = L / n_t;
   } else if (kGateUp && !std::is_same<T, float>::value) {
-    const int slot = blockIdx.x >> 3;
+    const int slot = pid >> 3;
     tt = slot % n_t;
-    q0 = slot / n_t * 8 + (blockIdx.x & 7);
+    q0 = slot / n_t * 8 + (pid & 7);
   } else {
-    tt = blockIdx.x / n_q;
-    q0 = blockIdx.x % n_q;
+    tt = pid / n_q;
+    q0 = pid % n_q;
   }
   const int wtile = q0 % a.n_wtiles, split = q0 / a.n_wtiles;
   const int e = a.tile_map[2 + 2 * tt], row0 = a.tile_map[3 + 2 * tt];
@@ -296,9 +301,10 @@ hipError_t launch_items(FfnArgs a, hipStream_t s) {
   a.n_wtiles = kGateUp ? (a.I + C::kW / 2 - 1) / (C::kW / 2) : (a.H + C::kW - 1) / C::kW;
   const long long items = static_cast<long long>(a.n_wtiles) * a.max_tiles * a.splits;
   if (items == 0) return hipSuccess;
-  if (items > 0x7fffffffll || a.tile_rows > C::kT) return hipErrorInvalidValue;
-  ffn_general_kernel<T, kGateUp, C>
-      <<<dim3(static_cast<unsigned>(items)), dim3(kThreads), 0, s>>>(a);
+  if (items > INT_MAX - kGridX || a.tile_rows > C::kT) return hipErrorInvalidValue;
+  const dim3 grid(static_cast<unsigned>(std::min<long long>(items, kGridX)),
+                  static_cast<unsigned>((items + kGridX - 1) / kGridX));
+  ffn_general_kernel<T, kGateUp, C><<<grid, dim3(kThreads), 0, s>>>(a);
   return hipGetLastError();
 }
 

@@ -188,3 +188,30 @@ def test_static_scratch_drops_the_splits(dev):
                                ids.int().contiguous(), 0, out)
     # the same products in fp32, summed in another order
     assert (out - want).norm() <= 1e-5 * want.norm()
+
+
+def test_more_items_than_one_grid_dimension_holds(dev):
+    """2^24 workgroups of 256 threads are past what HIP takes in one grid
+    dimension: the general kernel's items go over two."""
+    T, H, I = 4096 * 1023, 4, 8448
+    plan = _capi.make_plan(T, H, I, 1, 1, _capi.F32)
+    assert plan.max_tiles * (I // 32) > 1 << 24
+    if torch.cuda.mem_get_info()[0] < plan.workspace_bytes + (4 << 30):
+        pytest.skip(f"needs {plan.workspace_bytes >> 30} GiB of GPU memory")
+    banner(f"general {plan.max_tiles * (I // 32)} gate_up items")
+    w1, w2 = make_bank(1, H, I, torch.float32, seed=3)
+    x = torch.randn(4096, H, generator=torch.Generator().manual_seed(3))
+    xd, d1, d2 = x.to(dev).repeat(T // 4096, 1), w1[0].to(dev), w2[0].to(dev)
+    tw = torch.ones(T, 1, device=dev)
+    ids = torch.zeros(T, 1, dtype=torch.int32, device=dev)
+    out = torch.full((T, H), float("nan"), device=dev)
+    ws = torch.empty(plan.workspace_bytes, dtype=torch.uint8, device=dev)
+    _capi.fused_experts(xd, [d1.data_ptr()], [d2.data_ptr()], I, tw, ids, 0, out, ws)
+    torch.cuda.synchronize()
+    del ws
+    torch.cuda.empty_cache()
+    # a row's sums do not depend on its place: every repeat is the first one
+    assert torch.equal(out.view(-1, 4096 * H), out[:4096].reshape(1, -1).expand(T // 4096, -1))
+    ref = oracle.fused_experts(x, w1, w2, np.ones((4096, 1), np.float32),
+                               np.zeros((4096, 1), np.int64), activation=0)
+    assert oracle.max_rel(out[:4096].double().cpu().numpy(), ref) <= 1e-5
