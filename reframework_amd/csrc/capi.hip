@@ -40,10 +40,12 @@ constexpr int kMaxDevices = 64;
 // Average rows per active expert up to which 16-row weight-streaming tiles run.
 constexpr int kSkinnyRows = 10;
 // And up to which 128-row tile maps run the general kernel rather than the
-// persistent 128-row one (mid_sized): at 62 to 66 rows 16 experts of I 6400 gain
-// 2 % and fine-grained experts lose 1 %, at 75 the Mixtral shape gains 5 %,
-// I 6400 loses 1 %; at 94 to 100 rows 2 to 10 % are lost.
-constexpr int kMidRows = 64;
+// persistent 128-row one (mid_sized), by the bytes of the active experts'
+// weights: the persistent kernel's start and end of a launch weigh less the more
+// there is to stream (it reaches 3.5 to 5.1 TB/s of weights below 3 GB, 5.1 to 5.9
+// above), while the general one falls from 6.3 TB/s at 12 rows to 4.9 at 64.
+constexpr int kMidRows = 64, kMidRowsLarge = 40;
+constexpr double kMidLargeBytes = 3e9;
 
 size_t align256(size_t v) { return (v + 255) & ~static_cast<size_t>(255); }
 
@@ -125,10 +127,27 @@ bool needs_general(const moe355_plan* p, int K, int features, int k_per_split, c
 }
 
 // Whether a 128-row tile map runs the general kernel's 128-row instance rather
-// than the persistent 128-row kernel.
+// than the persistent 128-row kernel. Layers, persistent / general time, routing
+// uniform and Zipf 1.1:
+//  * up to 3 GB of weights (13 layers of 4 to 128 experts, H 1024 to 8192): 1.03 to
+//    1.3 and 1.01 to 1.2 at 11 to 56 rows; at 64 rows 0.995 to 1.26 and 1.00 to 1.16.
+//    Beyond 64 it loses (16 experts of I 6400 1 % at 75 rows, 2 to 10 % at 94 to 100). Of
+//    Zipf 1.6 and 2.0 only those 16 experts lose, 1 to 4 % at 50 to 64 rows.
+//  * above (8 layers of 16 to 256 experts, 3.2 to 22 GB): 1.02 to 1.16 and 1.04 to
+//    1.13 up to 32 rows, 0.99 to 1.07 and 1.00 to 1.08 at 40, 0.92 to 0.99 and 0.94 to
+//    0.98 at 64.
+//  * above, and each matrix of a power of two of 2^23 elements or more (64, 32 and 16
+//    experts of H 4096 and I 2048, 4096, 8192): 0.95 to 1.00, 0.96 to 0.99 and 0.96 to
+//    1.05 at 12 to 40 rows of uniform routing. The general kernel streams 5.1 to 5.5
+//    TB/s there instead of 5.9 to 6.3; why was not traced.
 bool mid_sized(const moe355_plan* p) {
+  if (p->path != MOE355_PATH_MFMA_TILED128) return false;
   const long long act = std::min<long long>(p->E, p->rows);
-  return p->path == MOE355_PATH_MFMA_TILED128 && p->rows <= kMidRows * act;
+  const long long matrix = static_cast<long long>(p->H) * p->I;
+  int limit = kMidRows;
+  if (3.0 * act * matrix * elem_size(p->dtype) > kMidLargeBytes)
+    limit = matrix >= (1ll << 23) && !(matrix & (matrix - 1)) ? 0 : kMidRowsLarge;
+  return p->rows <= limit * act;
 }
 
 // Whether every weight row of K elements starts on a 128-byte line. Only then do

@@ -39,9 +39,9 @@
 // nothing with its barriers and epilogues and shares L2 between weights and
 // tokens), layers: Mixtral shape, 44 / 197 / 256 tokens 559 / 567 / 577 ->
 // 450 / 479 / 513 us; 16 experts of I 6400, 300 tokens 486 -> 444; 66 experts
-// top-8 of H 2048, I 1408, 128 / 300 tokens 249 / 256 -> 219 / 237. At about 75
-// rows per expert both take the same time, and above the persistent kernel
-// wins (mid_sized in capi.hip).
+// top-8 of H 2048, I 1408, 128 / 300 tokens 249 / 256 -> 219 / 237. Above some 40 to
+// 75 rows per expert, by the size of the layer, the persistent kernel wins
+// (mid_sized in capi.hip has the line and both sides of it).
 #include <algorithm>
 #include <climits>
 

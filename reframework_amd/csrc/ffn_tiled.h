@@ -577,7 +577,8 @@ void ffn_tiled16_kernel(const FfnArgs a) {
   wait_vmcnt<0>();
 }
 
-// 128-row token tiles (groups of about 64 to 104 rows; smaller ones run the
+// 128-row token tiles (groups of about 64 to 104 rows, of 40 and fewer in layers
+// of more than 3 GB of weights; mid_sized in capi.hip gives smaller ones to the
 // general kernel, ffn_general.hip, on the same maps). Few tokens meet
 // each weight slab, so a step carries a quarter of a full tile's MFMA work
 // (~256 cycles per sub-step) and the loads' latency shows. Token rows are

@@ -94,6 +94,33 @@ def test_128_row_maps_up_to_64_rows_per_expert(dts, I, m, dev):
     _check(gpu_fused(x, w1, w2, w, ids, path=path), x, w1, w2, w, ids, path=path)
 
 
+@pytest.mark.parametrize("E,H,I,T", [(24, 3072, 8192, 480), (24, 3072, 8192, 492),
+                                     (16, 4096, 8192, 96)])
+def test_128_row_maps_of_more_than_3_gb_of_weights(E, H, I, T, dev):
+    """Both sides of that dispatch: the general kernel up to 40 rows per expert,
+    the persistent one above and where a matrix is a power of two."""
+    K = 2
+    banner(f"128-row map E={E} H={H} I={I} T={T}")
+    plan = _capi.make_plan(T, H, I, E, K, _capi.BF16)
+    assert plan.path == _capi.PATH_MFMA_TILED128 and 6 * E * H * I > 3e9
+    g = torch.Generator(device=dev).manual_seed(T)
+    w1 = torch.empty(E, 2 * I, H, dtype=torch.bfloat16, device=dev).normal_(0, 0.02, generator=g)
+    w2 = torch.empty(E, H, I, dtype=torch.bfloat16, device=dev).normal_(0, 0.02, generator=g)
+    x = torch.empty(T, H, dtype=torch.bfloat16, device=dev).normal_(generator=g)
+    ids = torch.from_numpy(skewed_ids(T, K, E, seed=T, skew=1.0)).to(dev)
+    w = torch.rand(T, K, generator=g, device=dev)
+    out = fused_experts(x, w1, w2, w, ids)
+    want = torch.zeros(T, H, dtype=torch.float64, device=dev)
+    for e in range(E):
+        tok, slot = torch.nonzero(ids == e, as_tuple=True)
+        gate, up = (x[tok].double() @ w1[e].double().t()).chunk(2, -1)
+        y = (gate * torch.sigmoid(gate) * up) @ w2[e].double().t()
+        want.index_add_(0, tok, y * w[tok, slot, None].double())
+    # bf16 rounds the intermediate, the slot's result and the output once each
+    assert (out.double() - want).norm() <= 3 * 2.0 ** -9 * want.norm()
+    assert (out.double() - want).abs().max() <= 2e-2 * want.abs().max()
+
+
 @pytest.mark.parametrize("T", [3, 100])
 @pytest.mark.parametrize("dts,H,I", [("f32", 132, 68), ("bf16", 136, 200), ("f16", 256, 128)])
 def test_general_path_element_alignment(dts, H, I, T, dev):
