@@ -39,6 +39,9 @@ constexpr int kMaxDevices = 64;
 
 // Average rows per active expert up to which 16-row weight-streaming tiles run.
 constexpr int kSkinnyRows = 10;
+// In layers of at most kStreamSmallBytes of weights also beyond, while rows per
+// expert times those bytes stay below kStreamReadBytes (16 times what is read).
+constexpr double kStreamSmallBytes = 24e6, kStreamReadBytes = 500e6;
 // And up to which 128-row tile maps run the general kernel rather than the
 // persistent 128-row one (mid_sized), by the bytes of the active experts'
 // weights: the persistent kernel's start and end of a launch weigh less the more
@@ -226,10 +229,20 @@ int plan_impl(int T, int H, int I, int E, int K, int dtype, int path, bool compa
     // Sizes only the weight-streaming kernel tiles (H a multiple of 128 but not
     // of 256, or tokens past 2 GB) leave it for the general kernel at the same 10
     // rows (H 1152, I 3200, 8 experts top-2, 48 / 128 / 333 tokens: 53 / 97 / 198 us
-    // streaming, 48 / 53 / 78 general).
+    // streaming, 48 / 53 / 78 general), small layers later: while all that the
+    // 16-row tiles read of the weights, cached after the first, stays below some 30
+    // MB, their many short waves take less time than the general kernel's few
+    // workgroups (us, streaming / general: H 384, I 512, 16 experts, 11 and 24 rows
+    // per expert 20.0 / 23.1 and 22 / 23, 32 rows 27 / 23; H 896, I 512, 8 experts, 11 and
+    // 24 rows 23 / 26 and 25 / 26, 48 rows 31 / 29; H 384, I 384, 8 experts, 11, 48 and
+    // 100 rows 20 / 23, 22 / 24 and 30 / 25; H 384, I 1536, 8 experts (28 MB), 11 rows
+    // 22 / 22, 16 rows 26 / 23).
+    const double wbytes = 3.0 * act_e * H * I * esz;
+    const bool stream =
+        avg <= kSkinnyRows || (wbytes <= kStreamSmallBytes && avg * wbytes <= kStreamReadBytes);
     path = tiled_ok && avg > 104                  ? MOE355_PATH_MFMA_TILED
            : tiled_ok && avg > kSkinnyRows        ? MOE355_PATH_MFMA_TILED128
-           : skinny_ok && avg <= kSkinnyRows      ? MOE355_PATH_MFMA_SKINNY
+           : skinny_ok && stream                  ? MOE355_PATH_MFMA_SKINNY
                                                   : MOE355_PATH_SIMT;
   } else if (((path == MOE355_PATH_MFMA_TILED || path == MOE355_PATH_MFMA_TILED128) &&
               !tiled_ok) ||

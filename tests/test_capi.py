@@ -62,6 +62,16 @@ def test_plan_paths_and_layout(T, H, I, E, K, dtype, path):
         assert (I // 128) % p.down_splits == 0
 
 
+@pytest.mark.parametrize("E,H,I,rows,path", [
+    (8, 640, 1664, 10, _capi.PATH_MFMA_SKINNY), (8, 640, 1664, 11, _capi.PATH_SIMT),
+    (16, 384, 512, 26, _capi.PATH_MFMA_SKINNY), (16, 384, 512, 27, _capi.PATH_SIMT),
+    (8, 384, 384, 70, _capi.PATH_MFMA_SKINNY), (8, 384, 384, 71, _capi.PATH_SIMT),
+])
+def test_streaming_only_sizes_leave_it_by_rows_and_layer_size(E, H, I, rows, path):
+    # above 24 MB of weights at 10 rows per expert, below it at 500 MB / weights
+    assert _capi.make_plan(rows * E, H, I, E, 1, _capi.BF16).path == path
+
+
 def test_tiled_path_keeps_token_offsets_below_2gb():
     # token-row byte offsets are 32-bit with bit 31 marking padding rows
     assert _capi.make_plan(262143, 4096, 14336, 8, 2, _capi.BF16).path == _capi.PATH_MFMA_TILED

@@ -60,14 +60,20 @@ def test_general_path_group_sizes(m, dts, H, I, dev):
     _check(gpu_fused(x, w1, w2, w, ids, path=SIMT), x, w1, w2, w, ids, path=SIMT)
 
 
-@pytest.mark.parametrize("T,path,tile", [(40, _capi.PATH_MFMA_SKINNY, 16), (44, SIMT, 64),
-                                         (300, SIMT, 64)])
-def test_sizes_only_the_streaming_kernel_tiles(T, path, tile, dev):
-    # H a multiple of 128, not of 256: weight streaming up to 10 rows per expert
-    H, I, E, K = 384, 256, 4, 1
+@pytest.mark.parametrize("E,H,I,T,path,tile", [
+    # 25 MB of weights: weight streaming up to 10 rows per expert
+    (4, 640, 1664, 40, _capi.PATH_MFMA_SKINNY, 16), (4, 640, 1664, 44, SIMT, 64),
+    (4, 640, 1664, 300, SIMT, 64),
+    # 2.4 MB and 7.1 MB: up to 211 and 70 rows
+    (4, 384, 256, 44, _capi.PATH_MFMA_SKINNY, 16), (4, 384, 256, 847, _capi.PATH_MFMA_SKINNY, 16),
+    (4, 384, 256, 848, SIMT, 64), (8, 384, 384, 567, _capi.PATH_MFMA_SKINNY, 16),
+    (8, 384, 384, 568, SIMT, 64)])
+def test_sizes_only_the_streaming_kernel_tiles(E, H, I, T, path, tile, dev):
+    # H a multiple of 128, not of 256
+    K = 1
     plan = _capi.make_plan(T, H, I, E, K, _capi.BF16)
     assert (plan.path, plan.tile_rows) == (path, tile)
-    banner(f"H={H} T={T} path={path}")
+    banner(f"E={E} H={H} I={I} T={T} path={path}")
     w1, w2 = make_bank(E, H, I, torch.bfloat16, seed=T)
     x = torch.randn(T, H, generator=torch.Generator().manual_seed(T)).to(torch.bfloat16)
     ids = skewed_ids(T, K, E, seed=T, skew=0.5)
