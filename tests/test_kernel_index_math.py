@@ -4,16 +4,17 @@ Each kernel's work decomposition is replayed on the host with the kernel's
 own formulas, and every index it forms is checked against the buffer it
 addresses, before any of it runs on a GPU:
 
-  * permute (count_kernel + scatter_kernel, reframework_amd/csrc/permute.hip):
-    the scatter's LDS tables (`total`, `base`, the per-wave `wave_cnt`, the
-    per-part prefix sums over the count table) are replayed per block, round
-    and wave with every LDS word poisoned at kernel start, so a read of a word
-    the kernel never wrote fails; the ballot ranking
+  * permute (permute_one_kernel up to 1024 slots, count_kernel + scatter_kernel
+    above; reframework_amd/csrc/permute.hip): the LDS tables (`total`, `base`, the
+    per-wave `wave_cnt`, the scans, the per-part prefix sums over the count table)
+    are replayed per block, round and wave with every LDS word poisoned at kernel
+    start, so a read of a word the kernel never wrote fails; the ballot ranking
     is replayed bit by bit. Every slot_to_row / row_src write must stay in
     bounds, every row must be written once, and the result must equal the
-    oracle's stable grouping. A planted mistake (the per-round zeroing of
+    oracle's stable grouping. Planted mistakes (the per-round zeroing of
     `wave_cnt` covering only wave 0's row, which once sent row_src out of
-    bounds on the GPU) must be caught.
+    bounds on the GPU; in the one-block kernel, waves without slots leaving
+    their counts unwritten) must be caught.
   * the tiled grouped GEMM (ffn_tiled.h): the persistent schedule (XCD
     remap, work_split's K-split tail, decode_tile's per-expert item groups)
     must cover every (K-split, permuted row, weight tile) exactly once, by a
@@ -23,6 +24,18 @@ addresses, before any of it runs on a GPU:
     that the two token-loading waves fill) is a loaded row of the tile or a
     zero-filled padding row, and every valid row is read; token and weight
     offsets stay in their 32-bit buffer ranges.
+  * the general expert FFN (ffn_general.hip), which runs MOE355_PATH_SIMT above 10
+    rows per expert and most 128-row maps: its workgroups must take every
+    (K-split, weight tile, token tile) exactly once, a pair of weight tile and
+    split on one XCD where the launch deals them so; all loads must stay inside
+    their weight matrix and token tile and their K range, also those of the
+    steps prefetched past the last, and every chunk of the range must reach the
+    LDS once; every output element must be stored once, from rows that were
+    multiplied.
+  * the weight-streaming kernel's K walk (ffn_skinny.hip): loads of the plain and the
+    general instance inside their matrix and K range, every chunk multiplied once,
+    and in its pipelined loop every step issued before it is consumed, once, into a
+    free slot.
   * the weight-streaming kernel's in-kernel grouping (ffn_skinny.hip,
     group_slots): its outputs must equal the permute's, every LDS, meta and
     global index must stay in its array, and every tile it hands a workgroup
@@ -96,27 +109,124 @@ def _emulate_prefix(counts, b, E, parts_overrun=False):
     return total, base
 
 
+def _rank_in_wave(lanes):
+    """rank_in_wave on the 64 expert ids of a wave (-1: not routed): per lane its
+    rank among the lanes of the same expert and their number, by one ballot per
+    bit of the id."""
+    routed = lanes >= 0
+    bits = [((lanes >> bit) & 1).astype(bool) for bit in range(8)]
+    rank, same_n = np.zeros(WAVE, np.int64), np.zeros(WAVE, np.int64)
+    for ln in np.flatnonzero(routed):
+        same = routed.copy()
+        for bit in range(8):
+            same &= bits[bit] if bits[bit][ln] else ~bits[bit]
+        rank[ln], same_n[ln] = int(same[:ln].sum()), int(same.sum())
+    return rank, same_n
+
+
+def _wave_scan(E, values, out):
+    """wave_scan: lane l owns values l * per .. l * per + per - 1."""
+    per = -(-E // WAVE)
+    assert per <= 256 // WAVE
+    v = [[int(values[ln * per + i]) if i < per and ln * per + i < E else 0
+          for i in range(256 // WAVE)] for ln in range(WAVE)]
+    inc = np.cumsum([sum(x) for x in v])
+    for ln in range(WAVE):
+        ex = int(inc[ln]) - sum(v[ln])
+        for i in range(256 // WAVE):
+            if i < per and ln * per + i < E:
+                assert out[ln * per + i] == POISON
+                out[ln * per + i] = ex
+            ex += v[ln][i]
+    out[E] = int(inc[WAVE - 1])
+
+
+def emulate_permute_one(ids, E, tile_rows, max_tiles, emap=None, idle_waves_write=True):
+    """Replays permute_one_kernel (all slots in one block of SINGLE_MAX threads).
+    ``idle_waves_write`` False plants the mistake that waves without slots skip
+    the zeroing of their counts."""
+    T, K = ids.shape
+    R = T * K
+    assert R <= SINGLE_MAX
+    n_waves = SINGLE_MAX // WAVE
+    es = np.full(SINGLE_MAX, -1, np.int64)
+    es[:R] = _routed(ids.reshape(-1), emap, E)
+    wave_cnt = np.full((n_waves, 256), POISON, np.int64)
+    rank = np.zeros(SINGLE_MAX, np.int64)
+    for w in range(n_waves):
+        lanes = es[w * WAVE:(w + 1) * WAVE]
+        if idle_waves_write or (lanes >= 0).any():
+            for lane in range(WAVE):
+                for x in range(lane, E, WAVE):
+                    wave_cnt[w, x] = 0
+        rank[w * WAVE:(w + 1) * WAVE], n = _rank_in_wave(lanes)
+        for ln in range(WAVE):
+            if lanes[ln] >= 0 and rank[w * WAVE + ln] == 0:
+                wave_cnt[w, lanes[ln]] = n[ln]
+    total = np.full(256, POISON, np.int64)  # barrier; a thread per expert
+    for x in range(E):
+        assert (wave_cnt[:, x] != POISON).all(), "unwritten LDS read"
+        c = wave_cnt[:, x].copy()
+        wave_cnt[:, x] = np.concatenate([[0], np.cumsum(c)[:-1]])
+        total[x] = c.sum()
+    start = np.full(257, POISON, np.int64)  # barrier; wave 0 scans, the others order
+    _wave_scan(E, total, start)
+    order = np.full(256, POISON, np.int64)
+    for tid in range(WAVE, SINGLE_MAX):
+        for x in range(tid - WAVE, E, SINGLE_MAX):
+            r = sum(1 for f in range(E) if total[f] > total[x] or (total[f] == total[x] and f < x))
+            p = 2 * r if 2 * r < E else 2 * (E - 1 - r) + 1
+            assert 0 <= p < E and order[p] == POISON
+            order[p] = x
+    assert (order[:E] != POISON).all()
+    place_start = np.full(257, POISON, np.int64)  # barrier
+    _wave_scan(E, -(-total[order[:E]] // tile_rows), place_start)
+    slot_to_row = np.full(R, POISON, np.int64)
+    row_src = np.full(R, POISON, np.int64)
+    for tid in range(R):
+        e = es[tid]
+        row = int(start[e] + wave_cnt[tid // WAVE, e] + rank[tid]) if e >= 0 else -1
+        slot_to_row[tid] = row
+        if row >= 0:
+            assert row < R, f"row {row} outside [0, {R})"
+            assert row_src[row] == POISON, f"row {row} written twice"
+            row_src[row] = tid // K
+    nt = min(int(place_start[E]), max_tiles)  # barrier
+    tile_map = [nt, tile_rows]
+    for j in range(nt):
+        lo, hi = 0, E - 1
+        while lo < hi:
+            mid = (lo + hi + 1) >> 1
+            if place_start[mid] <= j:
+                lo = mid
+            else:
+                hi = mid - 1
+        e = int(order[lo])
+        h = tile_height(int(start[e + 1] - start[e]), tile_rows)
+        tile_map += [e, int(start[e] + (j - place_start[lo]) * h)]
+    return start[:E + 1].copy(), slot_to_row, row_src, tile_map
+
+
 def emulate_permute(ids, E, tile_rows, max_tiles, emap=None, zero_first_row_only=False):
-    """Replays count_kernel / scatter_kernel. Returns (offsets, slot_to_row,
+    """Replays permute_one_kernel or count_kernel / scatter_kernel. Returns (offsets, slot_to_row,
     row_src, tile_map); raises AssertionError on an out-of-bounds index, a
     row written twice or a read of unwritten LDS."""
+    if ids.size <= SINGLE_MAX:
+        return emulate_permute_one(ids, E, tile_rows, max_tiles, emap)
     T, K = ids.shape
     R = T * K
     e_of = _routed(ids.reshape(-1), emap, E)
-    n_blocks = 1 if R <= SINGLE_MAX else -(-R // CHUNK)
-    rounds = SINGLE_MAX // THREADS if n_blocks == 1 else CHUNK // THREADS
-    counts = np.zeros((n_blocks, E), np.int64)  # count_kernel (or the one block's own count)
+    n_blocks = -(-R // CHUNK)
+    rounds = CHUNK // THREADS
+    counts = np.zeros((n_blocks, E), np.int64)  # count_kernel
     for s in range(R):
         if e_of[s] >= 0:
-            counts[0 if n_blocks == 1 else s // CHUNK, e_of[s]] += 1
+            counts[s // CHUNK, e_of[s]] += 1
     slot_to_row = np.full(R, POISON, np.int64)
     row_src = np.full(R, POISON, np.int64)
     offsets = tile_map = None
     for b in range(n_blocks):
-        if n_blocks > 1:
-            total, base = _emulate_prefix(counts, b, E)
-        else:
-            total, base = counts[0].copy(), np.zeros(E, np.int64)
+        total, base = _emulate_prefix(counts, b, E)
         start = np.concatenate([[0], np.cumsum(total)])
         tiles = -(-total // tile_rows)
         tile_start = np.concatenate([[0], np.cumsum(tiles)])
@@ -141,8 +251,7 @@ def emulate_permute(ids, E, tile_rows, max_tiles, emap=None, zero_first_row_only
                 h = tile_height(int(start[e + 1] - start[e]), tile_rows)
                 tile_map += [e, int(start[e] + (j - place_start[lo]) * h)]
         wave_cnt = np.full((WAVES, 256), POISON, np.int64)  # LDS at kernel start
-        r = 0
-        while r < rounds and b * CHUNK + r * THREADS < R:
+        for r in range(rounds):
             # per-round zeroing, as the kernel indexes it
             for i in range(WAVES * E):
                 if zero_first_row_only:
@@ -154,17 +263,10 @@ def emulate_permute(ids, E, tile_rows, max_tiles, emap=None, zero_first_row_only
             rank = np.zeros(THREADS, np.int64)
             for w in range(WAVES):
                 lanes = es[w * WAVE:(w + 1) * WAVE]
-                routed = lanes >= 0
-                bits = [((lanes >> bit) & 1).astype(bool) for bit in range(8)]
+                rank[w * WAVE:(w + 1) * WAVE], same_n = _rank_in_wave(lanes)
                 for ln in range(WAVE):
-                    if not routed[ln]:
-                        continue
-                    same = routed.copy()
-                    for bit in range(8):
-                        same &= bits[bit] if bits[bit][ln] else ~bits[bit]
-                    rank[w * WAVE + ln] = int(same[:ln].sum())
-                    if rank[w * WAVE + ln] == 0:
-                        wave_cnt[w, lanes[ln]] = int(same.sum())
+                    if lanes[ln] >= 0 and rank[w * WAVE + ln] == 0:
+                        wave_cnt[w, lanes[ln]] = same_n[ln]
             for t in range(THREADS):
                 s = slots[t]
                 if s >= R:
@@ -184,7 +286,6 @@ def emulate_permute(ids, E, tile_rows, max_tiles, emap=None, zero_first_row_only
                 col = wave_cnt[:, ee]
                 assert (col != POISON).all(), "unwritten LDS read"
                 base[ee] += int(col.sum())
-            r += 1
     return offsets, slot_to_row, row_src, tile_map
 
 
@@ -240,6 +341,30 @@ def test_permute_emulation_catches_partial_wave_table_zeroing():
     ids = _finegrained_ids(700, 1)
     with pytest.raises(AssertionError):
         emulate_permute(ids, 66, 256, 10_000, zero_first_row_only=True)
+
+
+@pytest.mark.parametrize("T,K,E,drop", [(1, 1, 1, False), (65, 1, 1, False), (64, 1, 65, True),
+                                        (129, 1, 256, False), (127, 8, 200, True),
+                                        (1024, 1, 256, False), (128, 8, 256, True)])
+@pytest.mark.parametrize("tile_rows", [16, 64, 256])
+def test_one_block_permute_emulation_equals_oracle(T, K, E, drop, tile_rows):
+    ids = skewed_ids(T, K, E, seed=T * E, skew=1.0)
+    emap = [(-1 if e % 5 == 3 else e) for e in range(E)] if drop else None
+    o_off, o_s2r, o_src = oracle.permute(ids, E, emap)
+    offsets, s2r, src, tile_map = emulate_permute_one(ids, E, tile_rows, T * K, emap)
+    assert np.array_equal(offsets, o_off) and np.array_equal(s2r, o_s2r)
+    n = int(o_off[-1])
+    assert np.array_equal(src[:n], o_src[:n]) and (src[n:] == POISON).all()
+    counts = np.diff(o_off)
+    want = [(e, int(o_off[e]) + j * tile_height(int(counts[e]), tile_rows))
+            for e in tile_order(counts) for j in range(-(-int(counts[e]) // tile_rows))]
+    assert [tuple(tile_map[2 + 2 * j:4 + 2 * j]) for j in range(tile_map[0])] == want
+
+
+def test_one_block_permute_emulation_catches_unwritten_counts():
+    """Planted mistake: waves without slots leave their counts unwritten."""
+    with pytest.raises(AssertionError):
+        emulate_permute_one(_mixtral_ids(16), 8, 16, 100, idle_waves_write=False)
 
 
 def test_permute_prefix_emulation_catches_part_overrun():
@@ -458,10 +583,13 @@ def test_tiled_schedule_covers_once_in_bounds(name, T, H, I, E, make, gate_up):
     K = ids.shape[1]
     plan = _capi.make_plan(T, H, I, E, K, _capi.BF16)
     assert plan.path in (_capi.PATH_MFMA_TILED, _capi.PATH_MFMA_TILED128)
-    emulate_tiled(_counts(ids, E), plan, gate_up)
-    # the same routing on a forced 256-row tile map and a 128-row one
-    for path in (_capi.PATH_MFMA_TILED, _capi.PATH_MFMA_TILED128):
-        emulate_tiled(_counts(ids, E), _capi.make_plan(T, H, I, E, K, _capi.BF16, path), gate_up)
+    # the planned map, and the same routing on a forced 256-row map and a 128-row
+    # one; 128-row maps that the general kernel runs are replayed in both
+    for path in (-1, _capi.PATH_MFMA_TILED, _capi.PATH_MFMA_TILED128):
+        plan = _capi.make_plan(T, H, I, E, K, _capi.BF16, path)
+        emulate_tiled(_counts(ids, E), plan, gate_up)
+        if mid_sized(plan):
+            emulate_general(_counts(ids, E), plan, gate_up)
 
 
 @pytest.mark.parametrize("cus", [256, 80, 304])
@@ -472,6 +600,313 @@ def test_tiled_schedule_on_other_cu_counts(cus):
     plan = _capi.make_plan(3000, 4096, 2048, 16, 2, _capi.BF16)
     for gate_up in (True, False):
         emulate_tiled(_counts(ids, 16), plan, gate_up, cus=cus)
+
+
+# ----------------------------------------------------- general expert FFN
+GENERAL_ROW_BYTES = 128  # kRowBytes: bytes of one operand row per step
+GRID_X = 1 << 22         # kGridX
+
+
+def mid_sized(plan):
+    """capi.hip mid_sized: 128-row maps that the general kernel runs."""
+    if plan.path != _capi.PATH_MFMA_TILED128:
+        return False
+    act, matrix = min(plan.E, plan.rows), plan.H * plan.I
+    limit = 64
+    if 3.0 * act * matrix * 2 > 3e9:
+        limit = 0 if matrix >= 1 << 23 and matrix & (matrix - 1) == 0 else 40
+    return plan.rows <= limit * act
+
+
+def _k_per_split(plan, gate_up, step):
+    """k of one split: whole steps on MOE355_PATH_SIMT, the plan's even parts else."""
+    if gate_up:
+        return plan.H
+    if plan.path != _capi.PATH_SIMT:
+        assert plan.I % plan.down_splits == 0
+        return plan.I // plan.down_splits
+    return -(-(-(-plan.I // step)) // plan.down_splits) * step
+
+
+def general_decode(pids, n_t, n_q, gate_up16):
+    """(token tile, weight tile and split) of ffn_general_kernel's workgroups."""
+    if n_q % 8:
+        L = np.array([xcd_remap(int(p), n_t * n_q) for p in pids])
+        return L % n_t, L // n_t
+    if gate_up16:
+        slot = pids >> 3
+        return slot % n_t, slot // n_t * 8 + (pids & 7)
+    return pids // n_q, pids % n_q
+
+
+def emulate_general(counts, plan, gate_up, k_clamped=True):
+    """Replays one ffn_general_kernel launch over per-expert row counts.
+    ``k_clamped`` False plants the mistake that prefetches past the last step are
+    not clamped to it."""
+    f32 = plan.dtype == _capi.F32
+    esz = 4 if f32 else 2
+    N, chunks = 16 // esz, GENERAL_ROW_BYTES // 16
+    kW, kT, D = (64, 64, 1) if f32 else (128, 128, 2) if plan.tile_rows == 128 else (128, 64, 2)
+    assert plan.tile_rows == kT
+    NI, NX = kW // 32, kT // 32
+    E, H, I, R = plan.E, plan.H, plan.I, plan.rows
+    ld, nout = (H, I) if gate_up else (I, H)
+    splits = 1 if gate_up else plan.down_splits
+    n_wt = -(-I // (kW // 2)) if gate_up else -(-H // kW)
+    kps = _k_per_split(plan, gate_up, GENERAL_ROW_BYTES // esz)
+    offs = np.concatenate([[0], np.cumsum(counts)]).astype(np.int64)
+    tiles = [(e, int(offs[e]) + j * kT) for e in tile_order(counts)
+             for j in range(-(-int(counts[e]) // kT))]
+    assert len(tiles) <= plan.max_tiles
+
+    # the launch's grid, and every item taken once
+    launched = n_wt * plan.max_tiles * splits
+    gx, gy = min(launched, GRID_X), -(-launched // GRID_X)
+    assert gx * 256 < 1 << 32 and gy < 1 << 16 and gx * gy < 1 << 31
+    n_t, n_q = len(tiles), n_wt * splits
+    if n_t == 0:
+        return
+    assert n_t * n_q <= gx * gy
+    pids = np.arange(n_t * n_q)
+    tt, q = general_decode(pids, n_t, n_q, gate_up and not f32)
+    assert tt.min() >= 0 and tt.max() < n_t and q.min() >= 0 and q.max() < n_q
+    assert len(np.unique(tt * n_q + q)) == n_t * n_q
+    if n_q % 8 == 0:  # a pair's items share an XCD
+        assert ((pids & 7) == (q & 7)).all()
+
+    # K ranges: the splits tile [0, ld), each chunk of one loaded into the LDS once
+    lc = np.arange(chunks)
+    covered = np.zeros(ld // N, np.int64)
+    assert ld % N == 0 and kps % N == 0
+    last_off = 0
+    for split in range(splits):
+        kbeg = split * kps
+        kend = min(ld, kbeg + kps)
+        nchunks = (kend - kbeg) // N if kend > kbeg else 0
+        nsteps = -(-nchunks // chunks)
+        for st in range(nsteps + D if nsteps else 0):  # D steps are prefetched past the last
+            at = (min(st, nsteps - 1) if k_clamped else st) * chunks + lc
+            off = np.minimum(at, nchunks - 1) if k_clamped else at
+            assert (off >= 0).all() and kbeg + (off.max() + 1) * N <= kend
+            last_off = max(last_off, kbeg + int(off.max() + 1) * N)
+            if st < nsteps:
+                stored = st * chunks + lc < nchunks
+                assert (off[stored] == (st * chunks + lc)[stored]).all()
+                np.add.at(covered, kbeg // N + off[stored], 1)
+    assert (covered == 1).all() and last_off == ld
+
+    # rows and LDS places: 256 threads load 32 rows of 8 chunks a pass
+    def lds_at(r, c):
+        return r * GENERAL_ROW_BYTES + ((c ^ ((r >> 1) & 7)) << 4)
+
+    lrow = np.arange(256) // chunks
+    c = np.arange(256) % chunks
+    buf = set()
+    for qp in range((kW + kT) // 32):  # weight passes, then token passes
+        place = lds_at(lrow, c) + qp * 32 * GENERAL_ROW_BYTES
+        assert (place == lds_at(lrow + 32 * qp, c)).all()
+        buf.update(place.tolist())
+    assert buf == set(range(0, (kW + kT) * GENERAL_ROW_BYTES, 16))
+    f_of = np.zeros((n_wt, kW), np.int64)  # weight row of each tile row
+    for qp in range(kW // 32):
+        r = qp * 32 + np.arange(32)
+        for wt in range(n_wt):
+            f = wt * (kW // 2) + (r & (kW // 2 - 1)) if gate_up else wt * kW + r
+            f_of[wt, r] = np.minimum(f, nout - 1) + np.where(gate_up & (r >= kW // 2), I, 0)
+    assert f_of.min() >= 0 and f_of.max() < (2 * I if gate_up else H)
+
+    # MFMA operand rows and the outputs they make
+    lr, kq = np.arange(64) & 15, np.arange(64) >> 4
+
+    def w_row(wave_w, i):
+        if gate_up:
+            return wave_w * (kW // 4) + (i % (NI // 2)) * 16 + (kW // 2 if i >= NI // 2 else 0)
+        return wave_w * (kW // 2) + i * 16
+
+    feats = np.zeros((n_wt, kW), np.int64)
+    for wave_w in range(2):
+        for i in range(NI):
+            r0 = w_row(wave_w, i)
+            assert 0 <= r0 and r0 + 16 <= kW and r0 % 16 == 0
+            for h in range(2):
+                assert (lds_at(lr, 4 * h + kq) + r0 * GENERAL_ROW_BYTES == lds_at(r0 + lr, 4 * h + kq)).all()
+            if gate_up and i >= NI // 2:
+                assert r0 == w_row(wave_w, i - NI // 2) + kW // 2  # the matching up rows
+                continue
+            for wt in range(n_wt):
+                f = wt * (kW // 2 if gate_up else kW) + r0 + 4 * np.arange(4)
+                for f0 in f[f < nout]:
+                    assert f0 + 4 <= nout
+                    col = f0 - wt * (kW // 2 if gate_up else kW)
+                    assert (f_of[wt, col:col + 4] == np.arange(f0, f0 + 4)).all()
+                    feats[wt, col:col + 4] += 1
+    width = kW // 2 if gate_up else kW
+    used = np.arange(n_wt)[:, None] * width + np.arange(kW)[None, :]
+    assert (feats == ((used < nout) & (np.arange(kW) < width))).all()
+    done = np.zeros(R, np.int64)
+    for e, row0 in tiles:
+        row_end = min(row0 + kT, int(offs[e + 1]))
+        assert offs[e] <= row0 < row_end
+        loaded = np.minimum(row0 + np.arange(kT), row_end - 1)
+        assert (loaded >= row0).all()
+        J = (row_end - row0 + 31) // 32
+        J = 1 if J <= 1 else 2 if NX <= 2 or J == 2 else min(J, 4)
+        assert J <= NX
+        for wave_t in range(2):
+            for j in range(NX):
+                prow = row0 + (2 * j + wave_t) * 16 + np.arange(16)
+                stored = prow[prow < row_end]
+                if not len(stored):
+                    continue
+                # multiplied, and its block's rows among the J passes that were loaded
+                assert j < J and (j < J - 1 or row_end - row0 > 32 * (J - 1) + 16 * wave_t)
+                assert (loaded[stored - row0] == stored).all() and stored.max() - row0 < 32 * J
+                done[stored] += 1
+    assert (done[:int(offs[E])] == 1).all() and (done[int(offs[E]):] == 0).all()
+
+
+GENERAL_CASES = [
+    # H, I, E, K, T, dtype, path
+    (4, 4, 4, 2, 70, _capi.F32, -1), (132, 68, 4, 2, 300, _capi.F32, -1),
+    (1024, 2816, 8, 2, 512, _capi.F32, -1), (260, 324, 4, 2, 22, _capi.F32, -1),
+    (8, 8, 4, 2, 70, _capi.BF16, -1), (136, 200, 4, 2, 300, _capi.BF16, -1),
+    (264, 520, 4, 2, 70, _capi.F16, -1), (1240, 3304, 12, 3, 333, _capi.BF16, -1),
+    (72, 136, 4, 2, 129, _capi.F16, -1), (1152, 3200, 8, 2, 48, _capi.BF16, -1),
+    (4096, 14336, 8, 2, 197, _capi.F16, -1), (256, 128, 3, 1, 190, _capi.BF16, 4),
+    (256, 640, 3, 1, 98, _capi.F16, 4), (2048, 1408, 64, 6, 300, _capi.BF16, -1),
+    (512, 256, 128, 8, 600, _capi.BF16, -1), (256, 256, 256, 8, 1024, _capi.BF16, -1),
+]
+
+
+@pytest.mark.parametrize("gate_up", [True, False], ids=["gate_up", "down"])
+@pytest.mark.parametrize("H,I,E,K,T,dtype,path", GENERAL_CASES)
+def test_general_kernel_covers_once_in_bounds(H, I, E, K, T, dtype, path, gate_up):
+    plan = _capi.make_plan(T, H, I, E, K, dtype, path)
+    assert mid_sized(plan) or (plan.path == _capi.PATH_SIMT and plan.tile_rows == 64)
+    for skew in (0.0, 2.0):
+        counts = _counts(skewed_ids(T, K, E, seed=T, skew=skew), E)
+        emulate_general(counts, plan, gate_up)
+    dropped = counts.copy()
+    dropped[1::2] = 0  # experts of another rank
+    emulate_general(dropped, plan, gate_up)
+
+
+def test_general_kernel_emulation_catches_unclamped_prefetch():
+    """Planted mistake: the steps prefetched past the last are not clamped to it."""
+    plan = _capi.make_plan(300, 132, 68, 4, 2, _capi.F32)
+    counts = _counts(skewed_ids(300, 2, 4, seed=1, skew=1.0), 4)
+    with pytest.raises(AssertionError):
+        emulate_general(counts, plan, True, k_clamped=False)
+
+
+# ---------------------------------------------- weight-streaming kernel's K walk
+SKINNY_STEP_CHUNKS = 16  # kStepChunks
+
+
+def emulate_skinny_walk(plan, gate_up, general):
+    """Replays the loads of ffn_skinny_kernel for every row group and K-split
+    (chunks of 16 bytes; rows and chunks as the lanes address them)."""
+    esz = 4 if plan.dtype == _capi.F32 else 2
+    N = 16 // esz
+    step = SKINNY_STEP_CHUNKS * N
+    ld, nout = (plan.H, plan.I) if gate_up else (plan.I, plan.H)
+    splits = 1 if gate_up else plan.down_splits
+    kps = _k_per_split(plan, gate_up, step)
+    D = 2 if gate_up else 4
+    lane = np.arange(WAVE)
+    n_wt = -(-nout // 16)
+    if not general:
+        assert ld % step == 0 and kps % step == 0 and nout % 16 == 0 and kps * splits == ld
+    covered = np.zeros(ld // N, np.int64)
+    for split in range(splits):
+        kbeg = split * kps
+        nchunks = (min(kps, ld - kbeg) // N if kbeg < ld else 0) if general else kps // N
+        nsteps = -(-nchunks // SKINNY_STEP_CHUNKS)
+        for idx in range(nsteps):
+            left = nchunks - idx * SKINNY_STEP_CHUNKS
+            mult = np.zeros((16, SKINNY_STEP_CHUNKS), np.int64)
+            for j in range(4):
+                r = 4 * j + (lane >> 4)
+                c = (lane & 15) ^ r
+                src = np.minimum(c, left - 1)
+                assert (src >= 0).all() and (kbeg + (idx * SKINNY_STEP_CHUNKS + src + 1) * N <= ld).all()
+                # LDS place (64 j + lane) * 16 holds row r, logical chunk c
+                assert ((64 * j + lane) * 16 == r * 256 + ((c ^ r) << 4)).all()
+                ok = c < left
+                mult[r[ok], c[ok]] += 1
+            for s in range(4):  # tokens: logical chunk 4 s + lane / 16, as the MFMA reads the weights
+                c = 4 * s + (lane >> 4)
+                assert (kbeg + (idx * SKINNY_STEP_CHUNKS + np.minimum(c, left - 1) + 1) * N <= ld).all()
+                assert ((mult[lane & 15, c] == 1) == (c < left)).all()
+            k0 = kbeg // N + idx * SKINNY_STEP_CHUNKS
+            covered[k0:k0 + min(left, SKINNY_STEP_CHUNKS)] += 1
+        emulate_skinny_pipeline(nsteps, D)
+    assert (covered == 1).all()
+    for group in (0, n_wt - 1):
+        last_row = nout - 1 - group * 16
+        assert last_row >= 0
+        rows = group * 16 + np.minimum(np.arange(16), last_row)
+        assert rows.max() < nout
+        stored = 4 * np.arange(4)
+        stored = stored[stored <= last_row]
+        assert (group * 16 + stored + 4 <= nout).all()
+
+
+def emulate_skinny_pipeline(nsteps, D):
+    """The kernel's loops: every step issued into a free slot, consumed once."""
+    slots, consumed = [None] * D, []
+
+    def issue(d, st):
+        assert slots[d] is None and st < nsteps
+        slots[d] = st
+
+    def consume(d, st):
+        assert slots[d] == st
+        slots[d] = None
+        consumed.append(st)
+
+    st = 0
+    if nsteps >= 2 * D:
+        for d in range(D):
+            issue(d, d)
+        while True:
+            for d in range(D):
+                consume(d, st + d)
+                issue(d, st + d + D)
+            st += D
+            if not st + 2 * D <= nsteps:
+                break
+    else:
+        for d in range(D):
+            if d < nsteps:
+                issue(d, d)
+    while st < nsteps:
+        for d in range(D):
+            if st + d < nsteps:
+                consume(d, st + d)
+                if st + d + D < nsteps:
+                    issue(d, st + d + D)
+        st += D
+    assert consumed == list(range(nsteps)) and slots == [None] * D
+
+
+@pytest.mark.parametrize("D", [2, 4])
+def test_skinny_pipeline_consumes_every_step_once(D):
+    for nsteps in range(64):
+        emulate_skinny_pipeline(nsteps, D)
+
+
+@pytest.mark.parametrize("H,I,dtype,general", [
+    (4096, 14336, _capi.BF16, False), (2048, 1408, _capi.BF16, False), (1024, 2816, _capi.F32, True),
+    (4, 4, _capi.F32, True), (132, 68, _capi.F32, True), (260, 324, _capi.F32, True),
+    (8, 8, _capi.BF16, True), (136, 200, _capi.BF16, True), (264, 520, _capi.F16, True),
+    (1240, 3304, _capi.BF16, True), (512, 256, _capi.F32, False)])
+def test_skinny_k_walk_in_bounds(H, I, dtype, general):
+    for T, K, E in ((1, 2, 8), (16, 2, 8), (13, 4, 32)):
+        plan = _capi.make_plan(T, H, I, E, K, dtype)
+        assert plan.tile_rows == 16
+        for gate_up in (True, False):
+            emulate_skinny_walk(plan, gate_up, general)
 
 
 # --------------------------------------------------- skinny in-kernel grouping
@@ -592,24 +1027,32 @@ import _random_shapes  # noqa: E402
 def test_random_shapes_index_math_in_bounds(c):
     """The configurations of tests/test_gpu_random_shapes.py, replayed here
     first: the permute (or the in-kernel grouping at <= 64 slots) equal to the
-    oracle's grouping and in bounds, and the tiled schedules covering every
-    item once within their buffers."""
+    oracle's grouping and in bounds, and the items and loads of the kernel that
+    runs each covering everything once within their buffers."""
     T, K, E = c["T"], c["K"], c["E"]
     ids = skewed_ids(T, K, E, c["seed"], c["skew"])
     emap = c["emap"]
     plan = _capi.make_plan(T, c["H"], c["I"], E, K, _random_shapes.DTYPES[c["dt"]])
     o_off, o_s2r, _ = oracle.permute(ids, E, emap)
-    if plan.path == _capi.PATH_MFMA_SKINNY and plan.rows <= 64:
+    if plan.tile_rows == 16 and plan.rows <= 64:
         for t in range(plan.max_tiles):
             offsets, s2r, _, _, _ = emulate_group_slots(ids, E, plan.max_tiles, emap, ttile=t)
             assert np.array_equal(offsets, o_off) and np.array_equal(s2r, o_s2r)
     else:
         offsets, s2r, _, _ = emulate_permute(ids, E, plan.tile_rows, plan.max_tiles, emap)
         assert np.array_equal(offsets, o_off) and np.array_equal(s2r, o_s2r)
-    if plan.path in (_capi.PATH_MFMA_TILED, _capi.PATH_MFMA_TILED128):
-        counts = np.diff(o_off)
-        emulate_tiled(counts, plan, True)
-        emulate_tiled(counts, plan, False)
+    counts = np.diff(o_off)
+    for gate_up in (True, False):
+        if plan.tile_rows == 16:  # aligned operands: the general instance for partial steps only
+            esz = 4 if plan.dtype == _capi.F32 else 2
+            step = SKINNY_STEP_CHUNKS * 16 // esz
+            ld, kps = plan.H if gate_up else plan.I, _k_per_split(plan, gate_up, step)
+            emulate_skinny_walk(plan, gate_up, bool(
+                ld % step or kps % step or kps * (1 if gate_up else plan.down_splits) != ld))
+        elif plan.path == _capi.PATH_SIMT or mid_sized(plan):
+            emulate_general(counts, plan, gate_up)
+        else:
+            emulate_tiled(counts, plan, gate_up)
 
 
 def emulate_norm_router_tile(H, E, T, t0):
