@@ -1,8 +1,8 @@
 """The general expert-FFN path (MOE355_PATH_SIMT): fp32 layers and sizes the
 bf16/f16 tiled kernels do not take, at the edges of its tiles: 16-row tiles up
 to ten rows per expert and 64-row tiles above, K steps of 128 and 256 bytes,
-feature tiles of 16 to 128, against the fp64 oracle (the tolerances of the
-other paths' tests)."""
+feature tiles of 16 to 128, and the 128-row maps that its kernel shares with the
+tiled family, against the fp64 oracle (the tolerances of the other paths' tests)."""
 
 from __future__ import annotations
 
@@ -155,6 +155,78 @@ def test_general_path_element_alignment(dts, H, I, T, dev):
     _capi.down(plan, p2, ws)
     _capi.combine(plan, tw, out, False, ws)
     _check(out, x, w1, w2, w, ids, path=SIMT)
+
+
+@pytest.mark.parametrize("act", [1, 2], ids=["gelu", "gelu_tanh"])
+@pytest.mark.parametrize("T", [3, 70])
+@pytest.mark.parametrize("dts,H,I", [("f32", 132, 68), ("bf16", 136, 200), ("f16", 256, 144)])
+def test_general_path_activations(dts, H, I, T, act, dev):
+    E, K = 4, 2
+    dt = DT[dts]
+    banner(f"general {dts} T={T} activation {act}")
+    assert _capi.make_plan(T, H, I, E, K, _capi.dtype_code(dt)).path == SIMT
+    w1, w2 = make_bank(E, H, I, dt, seed=act)
+    x = torch.randn(T, H, generator=torch.Generator().manual_seed(T)).to(dt)
+    ids = skewed_ids(T, K, E, seed=T, skew=0.5)
+    w = np.random.default_rng(T).random((T, K)).astype(np.float32)
+    _check(gpu_fused(x, w1, w2, w, ids, act=act), x, w1, w2, w, ids, act=act)
+
+
+@pytest.mark.parametrize("T", [5, 70])
+@pytest.mark.parametrize("dts,H,I", [("f32", 132, 68), ("bf16", 136, 200)])
+def test_general_path_keeps_infinite_tokens_to_themselves(dts, H, I, T, dev):
+    """A token row ends inside a K step and the next one starts with infinities;
+    the last one is also what rows past the group read."""
+    dt = DT[dts]
+    E, K = 2, 1
+    banner(f"general {dts} infinite tokens T={T}")
+    w1, w2 = make_bank(E, H, I, dt, seed=5)
+    ids = np.zeros((T, K), np.int64)
+    w = np.ones((T, K), np.float32)
+    x = torch.randn(T, H, generator=torch.Generator().manual_seed(T)).to(dt)
+    ref = oracle.fused_experts(x, w1, w2, w, ids, activation=0)
+    bad = [1, T - 1]
+    x[bad, :4] = float("inf")
+    got = gpu_fused(x, w1, w2, w, ids).double().cpu().numpy()
+    assert not np.isfinite(got[bad]).any()
+    keep = np.setdiff1d(np.arange(T), bad)
+    assert oracle.max_rel(got[keep], ref[keep]) <= (1e-5 if dt == torch.float32 else 2e-2)
+
+
+def test_token_rows_past_2_gb(dev):
+    """Sizes of the tiled kernels whose tokens exceed their 32-bit offsets run
+    the general kernel above 10 rows per expert; tokens from both ends and the
+    2 GB boundary against the oracle."""
+    T, H, I, E, K = 131100, 8192, 128, 2, 1
+    banner(f"token rows past 2 GB T={T} H={H}")
+    plan = _capi.make_plan(T, H, I, E, K, _capi.BF16)
+    assert T * H * 2 > 1 << 31 and plan.path == SIMT and plan.tile_rows == 64
+    w1, w2 = make_bank(E, H, I, torch.bfloat16, seed=8)
+    x = torch.empty(T, H, dtype=torch.bfloat16, device=dev).normal_(
+        generator=torch.Generator(device=dev).manual_seed(8))
+    ids = np.random.default_rng(8).integers(0, E, (T, K))
+    w = np.random.default_rng(9).random((T, K)).astype(np.float32)
+    out = fused_experts(x, [t.to(dev) for t in w1], [t.to(dev) for t in w2],
+                        torch.from_numpy(w).to(dev), torch.from_numpy(ids).to(dev))
+    pick = np.r_[0:24, T // 2:T // 2 + 8, 131060:131100]
+    _check(out[pick], x[pick].cpu(), w1, w2, w[pick], ids[pick], path=SIMT)
+
+
+@pytest.mark.parametrize("skew", [1.1, 2.0])
+@pytest.mark.parametrize("T,E,K", [(512, 16, 2), (330, 64, 6)])
+def test_128_row_maps_with_popular_experts(T, E, K, skew, dev):
+    """Full tiles of popular experts beside tiles of a few rows, on 128-row maps
+    of at most 64 rows per expert on average."""
+    H, I = 256, 384
+    plan = _capi.make_plan(T, H, I, E, K, _capi.BF16)
+    assert plan.path == _capi.PATH_MFMA_TILED128 and T * K <= 64 * E
+    ids = skewed_ids(T, K, E, seed=T, skew=skew)
+    assert np.bincount(ids.ravel()).max() > 256
+    banner(f"128-row map E={E} T={T} Zipf {skew}")
+    w1, w2 = make_bank(E, H, I, torch.bfloat16, seed=T)
+    x = torch.randn(T, H, generator=torch.Generator().manual_seed(T)).to(torch.bfloat16)
+    w = np.random.default_rng(T).random((T, K)).astype(np.float32)
+    _check(gpu_fused(x, w1, w2, w, ids), x, w1, w2, w, ids)
 
 
 @pytest.mark.parametrize("T", [2, 60])
