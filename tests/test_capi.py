@@ -212,8 +212,7 @@ def test_a_device_that_is_not_a_gpu_has_no_stream(monkeypatch):
         monkeypatch.setattr(_capi.lib(), name, reached)
     monkeypatch.setattr(torch.cuda, "_lazy_init", lambda: None)
     monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
-    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda index: 0x1000 + index,
-                        raising=False)
+    monkeypatch.setattr(_capi, "_raw_stream", lambda index: 0x1000 + index)
     assert _capi.stream_handle(torch.device("cuda:3")) == 0x1003
     with pytest.raises(ValueError, match="cpu"):
         _capi.stream_handle(torch.device("cpu"))
