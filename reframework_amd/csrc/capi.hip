@@ -132,13 +132,13 @@ bool needs_general(const moe355_plan* p, int K, int features, int k_per_split, c
 // Whether a 128-row tile map runs the general kernel's 128-row instance rather
 // than the persistent 128-row kernel. Layers, persistent / general time, routing
 // uniform and Zipf 1.1:
-//  * up to 3 GB of weights (13 layers of 4 to 128 experts, H 1024 to 8192): 1.03 to
-//    1.3 and 1.01 to 1.2 at 11 to 56 rows; at 64 rows 0.995 to 1.26 and 1.00 to 1.16.
+//  * up to 3 GB of weights (16 layers of 4 to 128 experts, H 1024 to 8192): 1.01 to
+//    1.3 at 11 to 56 rows, 0.995 to 1.26 and 1.00 to 1.2 at 64.
 //    Beyond 64 it loses (16 experts of I 6400 1 % at 75 rows, 2 to 10 % at 94 to 100). Of
 //    Zipf 1.6 and 2.0 only those 16 experts lose, 1 to 4 % at 50 to 64 rows.
-//  * above (8 layers of 16 to 256 experts, 3.2 to 22 GB): 1.02 to 1.16 and 1.04 to
+//  * above (7 layers of 16 to 256 experts, 3.2 to 22 GB): 1.00 to 1.16 and 1.02 to
 //    1.13 up to 32 rows, 0.99 to 1.07 and 1.00 to 1.08 at 40, 0.92 to 0.99 and 0.94 to
-//    0.98 at 64.
+//    0.98 at 64; with 8 experts (H 6144, I 16384) 1.05 to 1.11 from 40 to 64.
 //  * above, and each matrix of a power of two of 2^23 elements or more (64, 32 and 16
 //    experts of H 4096 and I 2048, 4096, 8192): 0.95 to 1.00, 0.96 to 0.99 and 0.96 to
 //    1.05 at 12 to 40 rows of uniform routing. The general kernel streams 5.1 to 5.5
@@ -219,13 +219,15 @@ int plan_impl(int T, int H, int I, int E, int K, int dtype, int path, bool compa
                         2ll * I * H * esz < (1ll << 32);
   const bool skinny_ok = mfma && H % 128 == 0 && I % 128 == 0;
   if (path < 0) {
-    // Average rows per active expert decide (measured layer times, Mixtral,
-    // Phi-3.5 and fine-grained shapes): weight streaming with 16-token tiles up
-    // to 10 rows (beyond that each 16-row tile re-streams the weights), the
-    // 256-row kernel on 128-row tiles up to 104 rows (Mixtral 64 and 256
-    // tokens: 0.55 and 0.59 ms against 0.56 and 0.65 with 256-row tiles;
-    // fine-grained 512 tokens 0.31 against 0.32), 256-row tiles above
-    // (Mixtral 512 tokens: 0.67 against 0.68 ms).
+    // Average rows per active expert decide (experts alone, us; Mixtral shape, and
+    // 66 experts top-8 of H 2048, I 1408, two of them shared): weight streaming with
+    // 16-token tiles up to 10 rows, beyond which more and more experts re-stream
+    // their weights (streaming / 128-row maps: 8 rows 441 / 426 and 218 / 214, 10 rows
+    // 509 / 435 and 227 / 218, 16 and 15 rows 700 / 433 and 253 / 225; 10 was the line
+    // against the persistent kernel, the general one is ahead from about 8), 128-row
+    // maps up to 104 rows (mid_sized picks their kernel), 256-row maps above (128 /
+    // 256: 16 rows 434 / 619, 64 and 62 rows 510 / 584 and 263 / 301, 104 rows 624 /
+    // 624 and 316 / 334, 128 and 124 rows 747 / 630 and 315 / 337).
     // Sizes only the weight-streaming kernel tiles (H a multiple of 128 but not
     // of 256, or tokens past 2 GB) leave it for the general kernel at the same 10
     // rows (H 1152, I 3200, 8 experts top-2, 48 / 128 / 333 tokens: 53 / 97 / 198 us

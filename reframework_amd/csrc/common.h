@@ -166,12 +166,6 @@ __device__ __forceinline__ float wave_sum(float v) {
   return v;
 }
 
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, kWave));
-  return v;
-}
-
 // Rows per token tile of an expert of n rows in a tile map of tile_rows-row
 // tiles. 256-row tiles share the expert's rows evenly over its ceil(n / 256)
 // tiles, the height rounded up to the 32-row token-block pair the 256-row

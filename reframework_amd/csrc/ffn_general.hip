@@ -24,15 +24,16 @@
 // the way (in both operands: past a weight row lies the next one, whose values
 // may be infinite) and operands need not be 16-byte aligned.
 //
-// fp32 is bound by its MFMA rate (157 TFLOP/s, a sixteenth of bf16's; an
-// all-register probe holds 150; the MFMAs are busy 73 to 80 % of the cycles in
+// fp32 is bound by its MFMA rate (157 TFLOP/s, a sixteenth of bf16's; a large
+// library product reaches 153, an all-register probe 150; the MFMAs are busy 73 to 80 % of the cycles in
 // which a CU holds work) and by the last round of items, which is why its tile
 // is small. 16-bit sizes on this path are bound by the weight stream
 // and the LDS. Before, one kernel did both with fp32 FMAs on the VALU, one
 // element per LDS read (gate_up + down, 64 x 64 tiles, 16 k a step). Layers,
 // before -> now: fp32 H 1024, I 2816, 8 experts top-2, 512 tokens 1.04 -> 0.21 ms
 // (86 TFLOP/s), 128 tokens 0.88 -> 0.10 ms; bf16 H 1240, I 3304, 12 experts
-// top-3, 333 tokens 1.44 -> 0.121 ms, 60 tokens 1.27 -> 0.085 ms.
+// top-3, 333 tokens 1.44 -> 0.123 ms, 60 tokens 1.24 -> 0.084 ms (the activation's
+// expf and division are 1 % of it).
 //
 // Groups of 10 to 64 rows of the tiled sizes are bound by the weight stream.
 // Against the persistent 128-row kernel (one workgroup per CU, which overlaps
