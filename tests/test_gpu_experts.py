@@ -13,7 +13,7 @@ Reference: fused_experts (reframework/moe/fused.py:49-87). Bars:
     largest output; and the output follows that rounding of y, not the other
     one.
 Every kernel family (256- and 128-token-tile MFMA, skinny MFMA with split-K,
-fp32 SIMT) is driven, with ragged and empty expert groups, tile-boundary group
+the general path) is driven, with ragged and empty expert groups, tile-boundary group
 sizes, dropped slots and int64 ids; each MFMA family is also forced onto
 shapes the automatic choice would give another one.
 """
@@ -258,6 +258,22 @@ def test_tile_boundary_group_sizes(m, path, dev):
     ids[-1, 0] = 3
     w1, w2 = make_bank(E, H, I, torch.bfloat16, seed=m)
     x = torch.randn(T, H, generator=torch.Generator().manual_seed(1000 + m)).to(torch.bfloat16)
+    w = np.ones((T, 1), np.float32)
+    _check(gpu_fused(x, w1, w2, w, ids, path=path), x, w1, w2, w, ids, path=path)
+
+
+@pytest.mark.parametrize("m", [1, 31, 32, 33, 63, 64, 65, 96, 97, 127, 128, 129])
+@pytest.mark.parametrize("dts,I", [("bf16", 256), ("f16", 640)])
+def test_persistent_128_row_group_sizes(m, dts, I, dev):
+    # 200 tokens on expert 0, m on expert 1: over 64 rows per expert on average
+    # (up to 64 the general kernel runs 128-row maps)
+    dt, path = DT[dts], _capi.PATH_MFMA_TILED128
+    H, T = 256, 200 + m
+    assert T > 64 * 2
+    banner(f"persistent 128-row kernel {dts} I={I} group of {m}")
+    ids = (np.arange(T) >= 200).astype(np.int64)[:, None]
+    w1, w2 = make_bank(2, H, I, dt, seed=m)
+    x = torch.randn(T, H, generator=torch.Generator().manual_seed(2000 + m)).to(dt)
     w = np.ones((T, 1), np.float32)
     _check(gpu_fused(x, w1, w2, w, ids, path=path), x, w1, w2, w, ids, path=path)
 

@@ -285,13 +285,14 @@ def test_mixtral_decode_full_size(T, splits, mixtral, dev):
     _check_sampled(out.cpu(), x, m["w1"], m["w2"], w.cpu().numpy(), ids_h, list(range(T)))
 
 
-def test_mixtral_t256_sampled_tokens(mixtral, dev):
-    """Mixtral-8x7B layer, T=256 (~64 rows per expert): the automatic plan
-    takes the 256-row kernel on 128-row token tiles with a 2-way K-split down
-    projection, and the 112 x 8 gate_up items leave a 128-item last round
+@pytest.mark.parametrize("T", [256, 384])
+def test_mixtral_128_row_tiles_sampled_tokens(T, mixtral, dev):
+    """Mixtral-8x7B layer on 128-row token tiles with a 2-way K-split down
+    projection. T=256 (64 rows per expert) runs the general kernel; T=384 the
+    persistent one, whose 112 x 8 gate_up items leave a 128-item last round
     that is cut along K."""
     m = mixtral
-    T, H, I, E, K = 256, m["H"], m["I"], m["E"], m["K"]
+    H, I, E, K = m["H"], m["I"], m["E"], m["K"]
     rng = np.random.default_rng(17)
     ids = np.argsort(rng.random((T, E)), axis=1)[:, :K].astype(np.int64)
     counts = np.bincount(ids.ravel(), minlength=E)
