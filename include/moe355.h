@@ -174,9 +174,9 @@ int moe355_topk_from_logits(const float* logits, int T, int E, int K, int renorm
  * average rows per active expert (T*K / min(T*K, E)): up to 10 skinny, up to
  * 104 128-row token tiles, above it 256-row tiles; fp32 and sizes that the
  * family of their group size does not take run MOE355_PATH_SIMT, on 16-row tiles up to
- * 10 rows and 64-row tiles above. Small layers (at most 24 MB of weights) of sizes
- * that of the three only skinny takes stay skinny while rows times weights are
- * below 500 MB. */
+ * 10 rows and 64-row tiles above. Layers of at most 24 MB of weights, of sizes that
+ * of the three only skinny takes, keep 16-row tiles there while rows times weights
+ * are below 500 MB. */
 int moe355_make_plan(int T, int H, int I, int E, int K, int dtype, moe355_plan* plan);
 
 /* moe355_make_plan with the kernel family forced (`path` = MOE355_PATH_*, or -1

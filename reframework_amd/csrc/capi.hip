@@ -229,22 +229,12 @@ int plan_impl(int T, int H, int I, int E, int K, int dtype, int path, bool compa
     // 256: 16 rows 434 / 619, 64 and 62 rows 510 / 584 and 263 / 301, 104 rows 624 /
     // 624 and 316 / 334, 128 and 124 rows 747 / 630 and 315 / 337).
     // Sizes only the weight-streaming kernel tiles (H a multiple of 128 but not
-    // of 256, or tokens past 2 GB) leave it for the general kernel at the same 10
+    // of 256, or tokens past 2 GB) leave it for the general path at the same 10
     // rows (H 1152, I 3200, 8 experts top-2, 48 / 128 / 333 tokens: 53 / 97 / 198 us
-    // streaming, 48 / 53 / 78 general), small layers later: while all that the
-    // 16-row tiles read of the weights, cached after the first, stays below some 30
-    // MB, their many short waves take less time than the general kernel's few
-    // workgroups (us, streaming / general: H 384, I 512, 16 experts, 11 and 24 rows
-    // per expert 20.0 / 23.1 and 22 / 23, 32 rows 27 / 23; H 896, I 512, 8 experts, 11 and
-    // 24 rows 23 / 26 and 25 / 26, 48 rows 31 / 29; H 384, I 384, 8 experts, 11, 48 and
-    // 100 rows 20 / 23, 22 / 24 and 30 / 25; H 384, I 1536, 8 experts (28 MB), 11 rows
-    // 22 / 22, 16 rows 26 / 23).
-    const double wbytes = 3.0 * act_e * H * I * esz;
-    const bool stream =
-        avg <= kSkinnyRows || (wbytes <= kStreamSmallBytes && avg * wbytes <= kStreamReadBytes);
+    // streaming, 48 / 53 / 78 on 64-row tiles).
     path = tiled_ok && avg > 104                  ? MOE355_PATH_MFMA_TILED
            : tiled_ok && avg > kSkinnyRows        ? MOE355_PATH_MFMA_TILED128
-           : skinny_ok && stream                  ? MOE355_PATH_MFMA_SKINNY
+           : skinny_ok && avg <= kSkinnyRows      ? MOE355_PATH_MFMA_SKINNY
                                                   : MOE355_PATH_SIMT;
   } else if (((path == MOE355_PATH_MFMA_TILED || path == MOE355_PATH_MFMA_TILED128) &&
               !tiled_ok) ||
@@ -252,13 +242,23 @@ int plan_impl(int T, int H, int I, int E, int K, int dtype, int path, bool compa
     return fail(MOE355_EUNSUPPORTED, "path %d cannot run dtype %d with H=%d I=%d T=%d", path,
                 dtype, H, I, T);
   }
+  // Small layers of such sizes stay on 16-row tiles beyond 10 rows: while all that
+  // those read of the weights, cached after the first, stays below some 30 MB, their
+  // many short waves take less time than the 64-row tiles' few workgroups (us, 16 /
+  // 64 rows: H 384, I 512, 16 experts, 11 and 24 rows per expert 20.0 / 23.1 and 22 /
+  // 23, 32 rows 27 / 23; H 896, I 512, 8 experts, 11 and 24 rows 23 / 26 and 25 / 26, 48
+  // rows 31 / 29; H 384, I 384, 8 experts, 11, 48 and 100 rows 20 / 23, 22 / 24 and 30 / 25; H
+  // 384, I 1536, 8 experts (28 MB), 11 rows 22 / 22, 16 rows 26 / 23).
+  const double wbytes = 3.0 * act_e * H * I * esz;
+  const bool small_stream = skinny_ok && !tiled_ok && wbytes <= kStreamSmallBytes &&
+                            avg * wbytes <= kStreamReadBytes;
   p->path = path;
   const bool tiled = path == MOE355_PATH_MFMA_TILED || path == MOE355_PATH_MFMA_TILED128;
   p->tile_rows = path == MOE355_PATH_MFMA_TILED      ? 256
                  : path == MOE355_PATH_MFMA_TILED128 ? 128
                  : path == MOE355_PATH_MFMA_SKINNY   ? 16
-                 : avg <= kSkinnyRows && !compact    ? 16
-                                                     : 64;
+                 : (avg <= kSkinnyRows || small_stream) && !compact ? 16
+                                                                    : 64;
   p->max_tiles = R > 0 ? static_cast<int>((R + static_cast<long long>(act_e) * (p->tile_rows - 1)) /
                                           p->tile_rows)
                        : 0;
@@ -304,7 +304,7 @@ int plan_impl(int T, int H, int I, int E, int K, int dtype, int path, bool compa
         p->down_splits = s;
       }
     }
-  } else if (p->path == MOE355_PATH_MFMA_SKINNY) {
+  } else if (p->tile_rows == 16 && skinny_ok) {
     // Spread the down projection (H/16 row groups per tile) over >= 8192 waves,
     // at most 8 splits (Mixtral shape: 4 splits instead of 2 at 4 and 16
     // tokens, down 98 -> 91 and 140 -> 133 us; 16 splits at one token are

@@ -62,14 +62,19 @@ def test_plan_paths_and_layout(T, H, I, E, K, dtype, path):
         assert (I // 128) % p.down_splits == 0
 
 
-@pytest.mark.parametrize("E,H,I,rows,path", [
-    (8, 640, 1664, 10, _capi.PATH_MFMA_SKINNY), (8, 640, 1664, 11, _capi.PATH_SIMT),
-    (16, 384, 512, 26, _capi.PATH_MFMA_SKINNY), (16, 384, 512, 27, _capi.PATH_SIMT),
-    (8, 384, 384, 70, _capi.PATH_MFMA_SKINNY), (8, 384, 384, 71, _capi.PATH_SIMT),
+@pytest.mark.parametrize("E,H,I,rows,path,tile", [
+    (8, 640, 1664, 10, _capi.PATH_MFMA_SKINNY, 16), (8, 640, 1664, 11, _capi.PATH_SIMT, 64),
+    (16, 384, 512, 10, _capi.PATH_MFMA_SKINNY, 16), (16, 384, 512, 11, _capi.PATH_SIMT, 16),
+    (16, 384, 512, 26, _capi.PATH_SIMT, 16), (16, 384, 512, 27, _capi.PATH_SIMT, 64),
+    (8, 384, 384, 70, _capi.PATH_SIMT, 16), (8, 384, 384, 71, _capi.PATH_SIMT, 64),
+    (8, 512, 256, 11, _capi.PATH_MFMA_TILED128, 128),
 ])
-def test_streaming_only_sizes_leave_it_by_rows_and_layer_size(E, H, I, rows, path):
+def test_streaming_only_sizes_leave_16_row_tiles_by_rows_and_layer_size(E, H, I, rows, path, tile):
     # above 24 MB of weights at 10 rows per expert, below it at 500 MB / weights
-    assert _capi.make_plan(rows * E, H, I, E, 1, _capi.BF16).path == path
+    p = _capi.make_plan(rows * E, H, I, E, 1, _capi.BF16)
+    assert (p.path, p.tile_rows) == (path, tile)
+    if tile == 16:
+        assert (I // 128) % p.down_splits == 0  # whole K parts: the plain instance
 
 
 def test_tiled_path_keeps_token_offsets_below_2gb():

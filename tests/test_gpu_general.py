@@ -61,12 +61,12 @@ def test_general_path_group_sizes(m, dts, H, I, dev):
 
 
 @pytest.mark.parametrize("E,H,I,T,path,tile", [
-    # 25 MB of weights: weight streaming up to 10 rows per expert
+    # 25 MB of weights: 16-row tiles up to 10 rows per expert
     (4, 640, 1664, 40, _capi.PATH_MFMA_SKINNY, 16), (4, 640, 1664, 44, SIMT, 64),
     (4, 640, 1664, 300, SIMT, 64),
-    # 2.4 MB and 7.1 MB: up to 211 and 70 rows
-    (4, 384, 256, 44, _capi.PATH_MFMA_SKINNY, 16), (4, 384, 256, 847, _capi.PATH_MFMA_SKINNY, 16),
-    (4, 384, 256, 848, SIMT, 64), (8, 384, 384, 567, _capi.PATH_MFMA_SKINNY, 16),
+    # 2.4 MB and 7.1 MB: 16-row tiles up to 211 and 70 rows
+    (4, 384, 256, 40, _capi.PATH_MFMA_SKINNY, 16), (4, 384, 256, 44, SIMT, 16),
+    (4, 384, 256, 847, SIMT, 16), (4, 384, 256, 848, SIMT, 64), (8, 384, 384, 567, SIMT, 16),
     (8, 384, 384, 568, SIMT, 64)])
 def test_sizes_only_the_streaming_kernel_tiles(E, H, I, T, path, tile, dev):
     # H a multiple of 128, not of 256
@@ -128,7 +128,8 @@ def test_128_row_maps_of_more_than_3_gb_of_weights(E, H, I, T, dev):
 
 
 @pytest.mark.parametrize("T", [3, 100])
-@pytest.mark.parametrize("dts,H,I", [("f32", 132, 68), ("bf16", 136, 200), ("f16", 256, 128)])
+@pytest.mark.parametrize("dts,H,I", [("f32", 132, 68), ("bf16", 136, 200), ("f16", 256, 128),
+                                     ("bf16", 384, 256)])
 def test_general_path_element_alignment(dts, H, I, T, dev):
     """Weights and tokens one element off a 16-byte boundary."""
     dt = DT[dts]
